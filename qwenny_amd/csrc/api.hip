@@ -280,7 +280,63 @@ extern "C" int qh_mat_download(const qh_mat* m, void* codes, void* scales, void*
 // need whole sums in one workgroup (split 1).
 struct Partition {
     int tile_waves, waves, split, groups_per_wave, tiles_per_wave;
+    bool mid = false;  // mid_kernel takes the product
 };
+
+// mid_kernel's partition of a product of 9-48 tokens, false where skinny_kernel stays: wave columns of two tiles x wave
+// rows over K (each a group per step, two for int4) per workgroup, and the split of K over the grid (plain products
+// only, others need whole sums in one workgroup). Fitted to both kernels' times over 7 to 48 tokens, four formats and
+// 20 shapes (rows 1536-151936, K 1920-17408): 1.38x the speed of skinny_kernel in the geometric mean, 0.4% off the best
+// partition of each case. Sides measured, us (plain: with add_rmsnorm):
+// - plain int4: skinny_kernel's 4-group splits are ahead up to 16 tokens while their partials are few ((5120, 6144) at
+//   9 / 16 / 24 tokens 11.9 / 13.2 / 14.5 against 13.1 / 13.2 / 13.6; (5120, 17408) 21.7 / 24.8 / 30.7 against 20.2 /
+//   20.5 / 21.2), and above 32 tokens (17.9 against 19.5: two token blocks leave two waves per SIMD). Per-channel and
+//   grouped int8 up to 16 tokens likewise ((4096, 2560) at 9 10.6 against 10.8), but not on small matrices, and bf16
+//   (one group per skinny wave, a partial each) never.
+// - whole sums: skinny_kernel where its 16-tile workgroups of 8-16 waves fill the chip, from 2000 tiles (int4 up to 16
+//   tokens 27.6 against 29.9; argmax above 32 tokens); below that its few workgroups leave the chip idle (4096 x 2560
+//   whole rows 16-34 against 8-16).
+// - wave rows: as many as give about 16 waves per CU (tiles x rows / 2), which smaller matrices need more of.
+static bool mid_partition(const qh_ctx* ctx, const qh_mat* m, size_t tokens, bool plain, bool argmax, Partition* out) {
+    if (tokens <= 8 || tokens > (size_t)SKINNY_MAX_M) return false;
+    // (tuning overrides of skinny_kernel's partition)
+    if (ctx->skinny_tile_waves || ctx->skinny_plain_wk != 1 || ctx->skinny_few) return false;
+    const int T = (int)(m->rows / TILE), G = (int)(m->cols / QG), M = (int)tokens;
+    const bool wide = is_i8(m->wt) || is_bf16(m->wt);  // formats of one group per wave and step
+    int wt, wk;
+    if (plain) {
+        const bool small = wide && (T <= 128 || (is_bf16(m->wt) && G < 32 && M <= 16));
+        if (!wide && (M > 32 || (M <= 16 && G < 96))) return false;
+        if (is_i8(m->wt) && M <= 16 && G < 64 && !small) return false;
+        wk = small ? 4 : 1;
+        if (small) wt = 1;
+        else if (!wide) wt = T >= 256 ? 8 : 4;
+        else wt = M > 32 || (T >= 256 && G < 32) ? 8 : 4;
+    } else if (wide) {
+        if (M > 32 && argmax) return false;
+        if (T <= 512) wt = 1, wk = M > 32 ? 4 : 8;
+        else if (T <= 1536) wt = M > 32 ? 4 : M > 24 ? 2 : 1, wk = M > 24 ? 2 : 4;
+        else wt = T <= 3000 || M > 32 ? 2 : 4, wk = 2;
+    } else {
+        if (T > 2000 && (M <= 16 || M > 32)) return false;
+        if (M > 32 && argmax) return false;
+        if (T <= 512) wt = M > 24 ? 2 : 1, wk = M > 32 ? 2 : M > 16 ? 4 : 8;
+        else if (T <= 1536) wt = 4, wk = 2;
+        else if (T <= 4096) wt = M > 24 ? 4 : 2, wk = 2;
+        else wt = 4, wk = M > 24 ? 2 : 1;
+    }
+    int split = 1;
+    if (plain) {
+        // workgroups the launch aims for: about 1000-1900 waves
+        const int aim = wt == 1 ? 384 : wt == 8 ? 240 : wide ? 384 : 256;
+        const int per = wk * (wide ? 1 : 2), steps = (G + per - 1) / per, columns = (T + 2 * wt - 1) / (2 * wt);
+        const int want = std::max(1, std::min(steps, (aim + columns - 1) / columns));
+        const int each = (steps + want - 1) / want;  // steps per split
+        split = (steps + each - 1) / each;
+    }
+    *out = Partition{wt, wt * wk, split, wide ? 1 : 2, SKINNY_TILES, true};
+    return true;
+}
 
 // The skinny kernel's partition of a product of m tokens (kernels.hip skinny_kernel): each wave takes SKINNY_TILES
 // tiles (plain int8 and bf16 products of 1-2 tokens: one) and 4 groups (1 when the group count is not a multiple of 4); a
@@ -291,7 +347,9 @@ struct Partition {
 // partials the consumer sums). Other epilogues need whole sums in one workgroup: its wave rows split K (reduced
 // through LDS), as few as give the launch enough waves to fill the CUs, dividing the chunks evenly and fitting the wave
 // and LDS limits; longer K is walked in super-chunks.
-static Partition skinny_partition(const qh_ctx* ctx, const qh_mat* m, size_t tokens, bool plain) {
+static Partition skinny_partition(const qh_ctx* ctx, const qh_mat* m, size_t tokens, bool plain,
+                                  bool argmax = false) {
+    if (Partition p; mid_partition(ctx, m, tokens, plain, argmax, &p)) return p;
     const int tiles = (int)(m->rows / TILE), G = (int)(m->cols / QG);
     // tiles per wave: one for plain int8 and bf16 products of 1-2 tokens (8 KiB of one tile, half the registers of a
     // two-tile wave, 5 waves per SIMD for int8: same-box graph replays, int8 per channel 27B set at M = 1 5.39 -> 5.49
@@ -388,7 +446,8 @@ static Launch make_launch(const qh_ctx* ctx, const qh_mat* w, const void* x, siz
     l.whole = whole;
     l.skinny = use_skinny(ctx, w, m, epi, whole);
     if (l.skinny) {
-        Partition p = skinny_partition(ctx, w, m, epi == QH_EPI_PLAIN && !whole);
+        Partition p = skinny_partition(ctx, w, m, epi == QH_EPI_PLAIN && !whole, epi == QH_EPI_ARGMAX);
+        l.mid = p.mid;
         l.tile_waves = p.tile_waves;
         l.waves = p.waves;
         l.split = p.split;

@@ -38,6 +38,7 @@ struct Launch {
     int groups_per_wave;    // skinny kernel: 4, or 1 when the group count is not a multiple of 4
     int tiles_per_wave;     // skinny kernel: SKINNY_TILES, or 1 (plain int8 and bf16 products of 1-2 tokens)
     int nc;                 // skinny kernel: super-chunks of K (groups / (wave rows x groups_per_wave)); set at launch
+    int mid;                // mid_kernel takes the product (9-48 tokens)
     int stage_out;          // skinny kernel, plain products: partials written through LDS in 16-byte row runs
     int cus;                // compute units (the prefill shape choice)
     int pf_shape;           // prefill workgroup shape: 0 chosen by size, else forced (kernels.hip prefill_epi)

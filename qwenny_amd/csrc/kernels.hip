@@ -1709,6 +1709,8 @@ static hipError_t skinny_nr(const Launch& l) {
         return l.groups_per_wave == 4 ? skinny_ng<F, EPI, NR, 4, TB>(l) : skinny_ng<F, EPI, NR, 1, TB>(l);
 }
 
+#include "mid.h"
+
 // Waves per workgroup of the workgroup-per-tile-pair kernels for nc chunks of K: a wave per 4-group chunk up to 8,
 // beyond that the chunks dealt out in turn. Eight-wave workgroups fill a CU's 24 wave slots (6 waves per SIMD) with
 // three workgroups, where 10- or 5-wave ones leave 4 idle. Same-box graph replays, us per whole-row product, against
@@ -1809,6 +1811,7 @@ static hipError_t skinny_epi(const Launch& l) {
             return hipGetLastError();
         }
     }
+    if (l.mid) return mid_epi<F, EPI>(l);
     if (l.m > 32) return skinny_nr<F, EPI, 4, 3>(l);
     if (l.m > 16) return skinny_nr<F, EPI, 4, 2>(l);
     // accumulator rows per lane: ceil(m / 4), at least 2 from 2 tokens (one row is the one-token form); same-box A/B
