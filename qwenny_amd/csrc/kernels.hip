@@ -1028,16 +1028,33 @@ static __global__ __launch_bounds__(512) void skinny_mt_kernel(MtArgs a) {
 }
 
 // ---------------------------------------------------------------------------------------------------------------
-// skinny_mw_kernel: whole rows (split 1) of a plain product of 2-8 tokens, int4 with bf16 scales, symmetric or with
-// zero points, no adapter: skinny_m1w_kernel's partition (a workgroup per tile pair over all of K, each wave taking
-// every WK-th chunk of 4 groups) with skinny_mt_kernel's arithmetic and token rows (each wave stages its tokens' rows
-// of its chunk, 16 bytes apart; token 4 r + lane / 16 in row r of a lane's accumulators). The waves' sums meet in LDS
-// and the first wave adds them in wave order (the 27B step at M = 5 with whole rows 0.3268 -> 0.3243 ms with the
-// token rows above).
-template <bool ZP, int NR>
-static __global__ __launch_bounds__(1024) void skinny_mw_kernel(MtArgs a) {
+// skinny_mw_kernel: products of 1-8 tokens (some of up to 16, skinny_epi) that need whole sums (plain products asked for whole rows, the SwiGLU
+// epilogue), with or without an adapter: skinny_m1w_kernel's partition (a workgroup per tile pair over all of K, each
+// wave taking every WK-th chunk of NG groups, 8 KiB of codes in flight) with skinny_mt_kernel's token rows (each wave
+// stages its tokens' rows of its chunk, 16 bytes apart; token 4 r + lane / 16 in row r of a lane's accumulators). The
+// waves' sums meet in LDS and are added in wave order. A last chunk of fewer than NG groups reads its last group again.
+// HBM-bound, and latency-bound in skinny_kernel, whose workgroups of 2-8 wave columns are few on matrices of this size
+// and walk K one staged super-chunk after another.
+struct MwArgs {
+    const u32x4* codes;
+    const void* scales;
+    const uint16_t* zeros;  // F_ZP only
+    const __bf16* x;
+    int ldx;
+    void* y;  // plain: f32 [m][tiles * 16]; SwiGLU: bf16 [m][tiles * 8]
+    int tiles, G, m;
+    uint32_t mask, magic;
+};
+struct NoLora {};
+
+// groups per chunk: 8 KiB of two tiles' codes
+template <int F>
+__host__ __device__ constexpr int mw_ng() { return 4 / CodeWords<F>::N; }
+
+template <int F, int EPI, int NR, bool LORA>
+static __global__ __launch_bounds__(512) void skinny_mw_kernel(MwArgs a, std::conditional_t<LORA, Launch, NoLora> ll) {
     extern __shared__ __attribute__((aligned(16))) uint8_t smem[];
-    constexpr int XP = mt_xpitch<4>();
+    constexpr int NG = mw_ng<F>(), XP = mt_xpitch<NG>(), CW = CodeWords<F>::N;
     const int lane = threadIdx.x & 63, wk = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     const int WK = blockDim.x >> 6;
     const int l16 = lane & 15, kq = lane >> 4;
@@ -1057,47 +1074,94 @@ static __global__ __launch_bounds__(1024) void skinny_mw_kernel(MtArgs a) {
         for (int r = 0; r < NR; r++) acc[t][r] = 0.0f;
     // MFMA row l16 holds token 4 (l16 % 4) + l16 / 4; rows past M read row M - 1 (never stored)
     const __bf16* xrow0 = xw + min(((l16 & 3) << 2) | (l16 >> 2), M - 1) * XP + 8 * kq;
-    for (int gw = 4 * wk; gw < G; gw += 4 * WK) {
+    for (int gw = NG * wk; gw < G; gw += NG * WK) {
+        const int col = min(gw * QG + 8 * lane, G * QG - 8);
         for (int r = 0; r < M; r++)
-            __builtin_amdgcn_global_load_lds((const void*)(a.x + (size_t)r * a.ldx + (size_t)gw * QG + 8 * lane),
-                                             (__attribute__((address_space(3))) void*)(xw + r * XP), 16, 0, 0);
+            if (NG == 4 || lane < 16 * NG)
+                __builtin_amdgcn_global_load_lds((const void*)(a.x + (size_t)r * a.ldx + col),
+                                                 (__attribute__((address_space(3))) void*)(xw + r * XP), 16, 0, 0);
         __builtin_amdgcn_sched_barrier(0);
-        uint32_t sraw[2][2], zraw[2];
+        uint32_t sraw[2][NG], zraw[2];  // scales: f32, or (int4) bf16 pairs
 #pragma unroll
-        for (int t = 0; t < 2; t++) {
-            const unsigned long long v =
-                __builtin_nontemporal_load((const unsigned long long*)(a.scales + scale_idx(tl[t], T, gw, l16)));
-            sraw[t][0] = (uint32_t)v, sraw[t][1] = (uint32_t)(v >> 32);
-            if (ZP) zraw[t] = __builtin_nontemporal_load(a.zeros + zero_idx(tl[t], T, gw, l16));
+        for (int t = 0; t < 2 && !(F & F_BF16); t++) {
+            const size_t si = scale_idx(tl[t], T, gw, l16);
+            if constexpr (NG == 4 && !(F & F_S32)) {
+                const unsigned long long v =
+                    __builtin_nontemporal_load((const unsigned long long*)((const uint16_t*)a.scales + si));
+                sraw[t][0] = (uint32_t)v, sraw[t][1] = (uint32_t)(v >> 32);
+            } else if constexpr (NG == 4) {
+                const u32x4 v = __builtin_nontemporal_load((const u32x4*)((const float*)a.scales + si));
+#pragma unroll
+                for (int i = 0; i < 4; i++) sraw[t][i] = v[i];
+            } else {  // int8: two f32
+                const unsigned long long v =
+                    __builtin_nontemporal_load((const unsigned long long*)((const float*)a.scales + si));
+                sraw[t][0] = (uint32_t)v, sraw[t][NG - 1] = (uint32_t)(v >> 32);
+            }
+            if (F & F_ZP) zraw[t] = __builtin_nontemporal_load(a.zeros + zero_idx(tl[t], T, gw, l16));
         }
-        u32x4 code[4][2];
+        u32x4 code[NG][2][CW];
 #pragma unroll
-        for (int gi = 0; gi < 4; gi++)
+        for (int gi = 0; gi < NG; gi++)
 #pragma unroll
             for (int t = 0; t < 2; t++)
-                code[gi][t] = __builtin_nontemporal_load(a.codes + ((size_t)tl[t] * G + gw + gi) * 64 + lane);
+#pragma unroll
+                for (int h = 0; h < CW; h++)
+                    code[gi][t][h] = __builtin_nontemporal_load(
+                        a.codes + (((size_t)tl[t] * G + min(gw + gi, G - 1)) * CW + h) * 64 + lane);
         // the activations landed (the weight loads issued after them may stay in flight)
-        constexpr int WL = 2 + (ZP ? 2 : 0) + 8;
+        constexpr int WL = ((F & F_BF16) ? 0 : 2) + ((F & F_ZP) ? 2 : 0) + 2 * NG * CW;
         __builtin_amdgcn_s_waitcnt((WL & 15) | ((WL >> 4) << 14) | (7 << 4) | (15 << 8));
 #pragma unroll
-        for (int gi = 0; gi < 4; gi++) {
+        for (int gi = 0; gi < NG; gi++) {
+            if (NG > 1 && gw + gi >= G) break;  // wave-uniform
             u32x4 xa[4];
 #pragma unroll
             for (int j = 0; j < 4; j++) xa[j] = *(const u32x4*)(xrow0 + gi * QG + 32 * j);
             f32x4 xsum = {0.0f, 0.0f, 0.0f, 0.0f};
 #pragma unroll
-            for (int j = 0; j < 4; j++) xsum = mfma(xa[j], ones, xsum);
+            for (int j = 0; j < 4 && !(F & F_BF16); j++) xsum = mfma(xa[j], ones, xsum);
 #pragma unroll
             for (int t = 0; t < 2; t++) {
+                auto frag = [&](int j) -> bf16x8 {
+                    if (F & F_BF16) return __builtin_bit_cast(bf16x8, code[gi][t][j % CW]);
+                    if (F & F_I8)
+                        return i8_biased(code[gi][t][(j >> 1) % CW][2 * (j & 1)], code[gi][t][(j >> 1) % CW][2 * (j & 1) + 1]);
+                    return i4_biased(code[gi][t][0][j], mask, magic);
+                };
                 f32x4 d = {0.0f, 0.0f, 0.0f, 0.0f};
 #pragma unroll
-                for (int j = 0; j < 4; j++) d = mfma(xa[j], i4_biased(code[gi][t][j], mask, magic), d);
-                const uint32_t w = sraw[t][gi >> 1];
-                const float sc = __uint_as_float((gi & 1) ? (w & 0xffff0000u) : (w << 16));
-                const float cz = ZP ? (float)(128 + (int)((zraw[t] >> (4 * gi)) & 15u)) : 136.0f;
+                for (int j = 0; j < 4; j++) d = mfma(xa[j], frag(j), d);
+                if (F & F_BF16) {  // the weights themselves
+#pragma unroll
+                    for (int r = 0; r < NR; r++) acc[t][r] += d[r];
+                    continue;
+                }
+                float sc;
+                if constexpr ((F & F_S32) != 0) {
+                    sc = __uint_as_float(sraw[t][gi]);
+                } else {
+                    const uint32_t w = sraw[t][gi >> 1];
+                    sc = __uint_as_float((gi & 1) ? (w & 0xffff0000u) : (w << 16));
+                }
+                const float cz = (F & F_ZP) ? (float)(128 + (int)((zraw[t] >> (4 * gi)) & 15u)) : (F & F_I8) ? 128.0f : 136.0f;
 #pragma unroll
                 for (int r = 0; r < NR; r++)
                     acc[t][r] = __builtin_fmaf(sc, __builtin_fmaf(-cz, xsum[r], d[r]), acc[t][r]);
+            }
+        }
+    }
+    if constexpr (LORA) {
+        if (wk == 0) {
+#pragma unroll
+            for (int t = 0; t < 2; t++) {
+                if (tile0 + t >= T) break;
+                f32x4 d = {0.0f, 0.0f, 0.0f, 0.0f};
+#pragma unroll
+                for (int r = 0; r < NR; r++) d[r] = acc[t][r];
+                lora_delta16<EPI == EPI_SILU>(ll, tile0 + t, 0, d);
+#pragma unroll
+                for (int r = 0; r < NR; r++) acc[t][r] = d[r];
             }
         }
     }
@@ -1109,15 +1173,40 @@ static __global__ __launch_bounds__(1024) void skinny_mw_kernel(MtArgs a) {
             if (tok < M) red[(wk * M + tok) * 32 + t * TILE + l16] = acc[t][r];
         }
     __syncthreads();
-    if (wk == 0) {
-        const int rows = T * TILE;
-        for (int i = lane; i < M * 32; i += 64) {
-            const int tok = i >> 5, row = i & 31, tile = tile0 + (row >> 4);
-            float v = 0.0f;
-            for (int c = 0; c < WK; c++) v += red[(c * M + tok) * 32 + row];
-            if (tile < T) __builtin_nontemporal_store(v, a.y + (size_t)tok * rows + tile * TILE + (row & 15));
+    // 32 rows per token, 2 tokens per wave and pass
+    for (int i = threadIdx.x; i < M * 32; i += 64 * WK) {
+        const int tok = i >> 5, row = i & 31, tile = tile0 + (row >> 4);
+        float v = 0.0f;
+        for (int c = 0; c < WK; c++) v += red[(c * M + tok) * 32 + row];
+        if (EPI == EPI_SILU) {
+            const float up = __shfl_xor(v, 8);  // rows 8..15 of a tile are the up rows of rows 0..7
+            if (tile < T && !(row & 8))
+                ((__bf16*)a.y)[(size_t)tok * T * (TILE / 2) + tile * (TILE / 2) + (row & 7)] = (__bf16)(silu(v) * up);
+        } else if (tile < T) {
+            __builtin_nontemporal_store(v, (float*)a.y + (size_t)tok * T * TILE + tile * TILE + (row & 15));
         }
     }
+}
+
+template <int F, int EPI>
+static hipError_t mw_launch(const Launch& l, int wk) {
+    constexpr int NG = mw_ng<F>();
+    const int tiles = l.rows / TILE;
+    const MwArgs a{(const u32x4*)l.codes, l.scales, l.zeros, (const __bf16*)l.x, l.ldx, l.y, tiles, l.cols / QG, l.m,
+                   l.nib_mask, l.bf16_magic};
+    const size_t lds = (size_t)wk * l.m * mt_xpitch<NG>() * 2 + (size_t)wk * l.m * 32 * 4;
+    const dim3 grid((tiles + 1) / 2), block(64 * wk);
+    auto go = [&](auto NRc) {
+        constexpr int NR = decltype(NRc)::value;
+        if (l.lora_rank) hipLaunchKernelGGL((skinny_mw_kernel<F, EPI, NR, true>), grid, block, lds, l.stream, a, l);
+        else hipLaunchKernelGGL((skinny_mw_kernel<F, EPI, NR, false>), grid, block, lds, l.stream, a, NoLora{});
+    };
+    // accumulator rows per lane: ceil(m / 4)
+    if (l.m <= 4) go(std::integral_constant<int, 1>{});
+    else if (l.m <= 8) go(std::integral_constant<int, 2>{});
+    else if (l.m <= 12) go(std::integral_constant<int, 3>{});
+    else go(std::integral_constant<int, 4>{});
+    return hipGetLastError();
 }
 
 // prefill_kernel
@@ -1726,15 +1815,15 @@ static int mw_waves(int nc) { return std::min(nc, 8); }
 template <int F, int EPI>
 static hipError_t skinny_epi(const Launch& l) {
     if constexpr (F == F_I4 || F == F_ZP) {
-        // Products that need whole sums of their rows, on the workgroup-per-tile-pair kernels (skinny_m1w_kernel at one
-        // token, skinny_mw_kernel for whole plain rows of 2-8 tokens): the one-token argmax, whole plain products, and
+        // One-token products that need whole sums of their rows, on skinny_m1w_kernel: the one-token argmax, whole plain products, and
         // the one-token SwiGLU product when K has at most 16 chunks of 4 groups. Same-box graph replays: the 27B
         // [gate; up] product (2 x 17408 rows, K 5120) 20.6 -> 18.9 us; the 27B head with its argmax, once the fold
         // became a launch of its own (while each workgroup counted itself done with a returning atomic, twice the
         // workgroups made it 20% slower), the headline step 0.2509 -> 0.2497 ms, and with keys[0] as the workgroups'
         // filter and target (no fold launch) 0.2495 ms against 0.2517 on another box (at 5 tokens the head on
         // skinny_mw_kernel made the step 0.2852 -> 0.3011 ms: it stays on skinny_kernel); whole plain products below
-        // the split product plus the sum of its partials (see qh_gemm's `whole`).
+        // the split product plus the sum of its partials (see qh_gemm's `whole`). Without an adapter; longer SwiGLU
+        // products take skinny_mw_kernel (2048 x 17408 24.7 -> 12.3 us).
         const int G = l.cols / QG;
         const bool fits = !l.lora_rank && G % 4 == 0 &&
                           ((EPI == EPI_ARGMAX && l.m == 1) || (EPI == EPI_PLAIN && l.split == 1) ||
@@ -1748,19 +1837,22 @@ static hipError_t skinny_epi(const Launch& l) {
                                a);
             return hipGetLastError();
         }
-        if constexpr (EPI == EPI_PLAIN) {
-            if (fits && l.m >= 2 && l.m <= 8) {
-                const int tiles = l.rows / TILE, nc = G / 4, wk = mw_waves(nc);
-                const MtArgs a{(const u32x4*)l.codes, (const uint16_t*)l.scales, l.zeros, (const __bf16*)l.x, l.ldx,
-                               (float*)l.y, tiles, G, l.m, l.nib_mask, l.bf16_magic};
-                const size_t lds = (size_t)wk * l.m * mt_xpitch<4>() * 2 + (size_t)wk * l.m * 32 * 4;
-                const dim3 grid((tiles + 1) / 2), block(64 * wk);
-                // accumulator rows per lane: ceil(m / 4)
-                if (l.m <= 4) hipLaunchKernelGGL((skinny_mw_kernel<F == F_ZP, 1>), grid, block, lds, l.stream, a);
-                else hipLaunchKernelGGL((skinny_mw_kernel<F == F_ZP, 2>), grid, block, lds, l.stream, a);
-                return hipGetLastError();
-            }
-        }
+    }
+    if constexpr (EPI != EPI_ARGMAX) {
+        // whole rows and SwiGLU products of up to 8 tokens, and of up to 16 where mid_kernel's or skinny_kernel's larger
+        // workgroups are few: up to 512 tiles, and up to 12 tokens to 1536 tiles and for int8. Same-box graph replays,
+        // us per product against skinny_kernel: SwiGLU at 1 / 2 / 5 / 8 tokens 34816 x 5120 int4 (18.0 on
+        // skinny_m1w_kernel) / 21.5 / 23.1 / 24.1 -> - / 18.7 / 19.7 / 21.5, int8 35.9 / 36.0 / 39.6 / 40.0 -> 31.0 /
+        // 30.8 / 32.3 / 33.5, 19456 x 2560 int4 - / 12.2 / 14.4 / 14.6 -> - / 8.0 / 8.7 / 9.0, int8 16.6 / 17.3 / 20.9 /
+        // 21.2 -> 11.4 / 11.4 / 13.1 / 13.5, bf16 20.1 / 21.0 / 28.7 / 28.8 -> 17.7 / 18.0 / 18.5 / 19.0; whole rows
+        // (5120, 6144) int8 12.5 / 13.4 / 33.3 / 33.9 -> 8.4 / 8.7 / 9.2 / 9.6, bf16 16.0 / 16.8 / 48.6 / 48.9 -> 11.5 /
+        // 11.6 / 12.1 / 12.7. Beyond 8 tokens against mid_kernel, at 9 / 12 / 16: 4864 x 2432 int4 7.2 / 7.8 / 8.0 ->
+        // 5.6 / 6.1 / 5.9, 19456 x 2560 13.1 / 13.0 / 13.2 -> 9.6 / 11.9 / 15.0, 34816 x 5120 27.6 / 28.7 / 29.0 ->
+        // 33.5 / 33.5 / 32.1 (its activations staged by every wave), int8 44.3 / 39.7 / 41.1 -> 34.7 / 36.8 / 46.0.
+        const int tiles = l.rows / TILE;
+        const int most = tiles <= 512 ? 16 : tiles <= 1536 || (F & F_I8) ? 12 : 8;
+        if (l.m <= most && (EPI == EPI_SILU || l.whole) && !l.xrows)
+            return mw_launch<F, EPI>(l, mw_waves((l.cols / QG + mw_ng<F>() - 1) / mw_ng<F>()));
     }
     if constexpr ((F == F_I4 || F == F_ZP) && EPI == EPI_PLAIN) {
         // the lean one-token kernel: the partition skinny_partition gives a plain one-token product (4 wave columns of

@@ -39,7 +39,6 @@ struct MidArgs {
     int gs_shift;
     uint32_t mask, magic;
 };
-struct MidNoLora {};
 
 // groups per wave and step: 4 KiB of codes of the wave's two tiles
 template <int F>
@@ -53,7 +52,7 @@ __host__ __device__ inline int mid_xbytes(int m, int gs_shift) { return ((m + 3)
 // (at least two waves per SIMD: the MFMA accumulators stay in VGPRs, as in skinny_m1_kernel)
 template <int F, int EPI, int TB, int WT, bool LORA>
 static __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2))) void mid_kernel(
-    MidArgs a, std::conditional_t<LORA, Launch, MidNoLora> ll) {
+    MidArgs a, std::conditional_t<LORA, Launch, NoLora> ll) {
     extern __shared__ __attribute__((aligned(1024))) uint8_t msmem[];
     constexpr int NG = mid_ng<F>(), CW = CodeWords<F>::N;
     const int lane = threadIdx.x & 63, wt = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
@@ -304,7 +303,7 @@ static hipError_t mid_launch(const Launch& l) {
         if constexpr (EPI != EPI_ARGMAX)
             hipLaunchKernelGGL((mid_kernel<F, EPI, TB, WT, true>), grid, block, lds, l.stream, a, l);
     } else {
-        hipLaunchKernelGGL((mid_kernel<F, EPI, TB, WT, false>), grid, block, lds, l.stream, a, MidNoLora{});
+        hipLaunchKernelGGL((mid_kernel<F, EPI, TB, WT, false>), grid, block, lds, l.stream, a, NoLora{});
     }
     hipError_t e = hipGetLastError();
     if (e == hipSuccess && EPI == EPI_ARGMAX) e = argmax_fold(l, l.m);

@@ -1,5 +1,5 @@
 """Products of 9-48 tokens on mid_kernel (whose partition depends on the matrix's tiles, groups and storage, and on the
-token count): odd tile counts and group counts, one tile, one group, both token blocks and their last rows, every
+token count) and whole sums of 1-16 tokens on skinny_mw_kernel: odd tile counts and group counts, one tile, one group, both token blocks and their last rows, every
 storage and epilogue, gathered logit rows. Products are exact products of the dequantized weights, so the bar is the
 decode kernels' 1e-4 against the f64 oracle (measured 1e-6: f32 sums of up to 2432 terms), one bf16 ulp beyond it for
 SwiGLU outputs."""
@@ -19,7 +19,10 @@ def _matrix(gemm, kind, n, k, silu=False):
     if kind == "bf16":
         w = f32_to_bf16(np.random.default_rng(n + k).standard_normal((n, k)).astype(np.float32) * 0.05)
         return Mat.new(gemm, w, k, silu=silu, int8=False), lambda x: bf16_to_f32(x).astype(np.float64) @ bf16_to_f32(w).T
-    q = make_quant(n + k, kind, n, k)
+    q = make_quant(n + k, kind[:2] if kind == "i4s32" else kind, n, k)
+    if kind == "i4s32":  # scales that bf16 does not hold
+        q.scales *= np.float32(1.001)
+        q.offsets[:] = -8 * q.scales
     return Mat.stack(gemm, [q], silu=silu), lambda x: oracle_y(q, x)
 
 
@@ -27,13 +30,13 @@ SHAPES = [(16, 128), (48, 2432), (528, 384), (2064, 1280), (4112, 640), (8208, 2
           (336, 12672)]
 
 
-@pytest.mark.parametrize("kind", ["i4", "i4z", "i8", "i8g", "bf16"])
+@pytest.mark.parametrize("kind", ["i4", "i4z", "i4s32", "i8", "i8g", "bf16"])
 @pytest.mark.parametrize("n,k", SHAPES)
 def test_plain_and_whole(gemm, kind, n, k):
     import torch
 
     mat, want_of = _matrix(gemm, kind, n, k)
-    for m in (9, 13, 16, 17, 25, 32, 33, 48):
+    for m in (1, 4, 5, 8, 9, 13, 16, 17, 25, 32, 33, 48):
         x = activations(m, "x", m, k)
         want = want_of(x)
         split = mat.split(m)
@@ -46,13 +49,13 @@ def test_plain_and_whole(gemm, kind, n, k):
             assert rel_err(y.double().sum(0).cpu().numpy(), want) <= 1e-4, (m, whole)
 
 
-@pytest.mark.parametrize("kind", ["i4", "i4z", "i8g", "bf16"])
+@pytest.mark.parametrize("kind", ["i4", "i4z", "i4s32", "i8g", "bf16"])
 @pytest.mark.parametrize("n,k", [(16, 384), (528, 1280), (8224, 384), (24608, 128), (33024, 256)])
 def test_silu(gemm, kind, n, k):
     import torch
 
     mat, want_of = _matrix(gemm, kind, n, k, silu=True)
-    for m in (9, 20, 32, 48):
+    for m in (1, 3, 8, 9, 12, 16, 20, 32, 48):
         print(f"mid silu {kind} {n}x{k} m={m}", flush=True)
         x = activations(m, "x", m, k)
         y = want_of(x)
@@ -88,7 +91,7 @@ def test_adapter(gemm):
     import torch
 
     n, k, rank = 1056, 1280, 16
-    for m in (12, 33):
+    for m in (1, 4, 7, 12, 33):
         rng = np.random.default_rng(m)
         xa = rng.standard_normal((2, m, 2 * rank)).astype(np.float32)
         b = (rng.standard_normal((n, rank)) * 0.1).astype(np.float16)
@@ -101,11 +104,12 @@ def test_adapter(gemm):
             dev = [torch.from_numpy(np.ascontiguousarray(v)).cuda()
                    for v in (xa, b.view(np.int16), np.asarray(tab, np.int32), slot, scale)]
             lora = (dev[0], 2, 2 * rank, dev[1], rank, dev[2], dev[3], dev[4])
-            y = torch.full((mat.split(m), m, n), float("nan"), device="cuda")
             if not silu:
-                gemm.run_lora(None, m, mat, to_dev(x), y, Epi.Plain, lora)
                 want = oracle.lora_add(want_of(x), xa, 2, b.view(np.uint16), rank, tab, slot, scale, m)
-                assert rel_err(y.double().sum(0).cpu().numpy(), want) <= 1e-4
+                for whole in (False, True):
+                    y = torch.full((1 if whole else mat.split(m), m, n), float("nan"), device="cuda")
+                    gemm.run_lora(None, m, mat, to_dev(x), y, Epi.Plain, lora, whole)
+                    assert rel_err(y.double().sum(0).cpu().numpy(), want) <= 1e-4, whole
                 continue
             out = torch.full((m, n // 2), float("nan"), dtype=torch.bfloat16, device="cuda")
             gemm.run_lora(None, m, mat, to_dev(x), out, Epi.Silu, lora)
