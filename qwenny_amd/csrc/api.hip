@@ -408,6 +408,21 @@ static bool use_skinny(const qh_ctx* ctx, const qh_mat* w, size_t m, int epi, in
     return !(m > 32 && fmt && w->rows * w->cols >= PF_FROM33_WEIGHTS);
 }
 
+// The splits of K of a plain product of m tokens on a dense bf16 matrix of few rows (mid.h narrow_launch), 0 for other
+// products: enough for about 512 workgroups, within the scratch the partials are kept in (one: none).
+static int narrow_split(const qh_ctx* ctx, const qh_mat* w, size_t m, int epi) {
+    const size_t tiles = w->rows / TILE;
+    if (epi != QH_EPI_PLAIN || !is_bf16(w->wt) || tiles > (size_t)NARROW_TILES || m <= (size_t)SKINNY_MAX_M ||
+        ctx->pf_shape || m > 65535 * 32)
+        return 0;
+    const int pairs = (int)(tiles + 1) / 2, wt = pairs >= 4 ? 4 : pairs >= 2 ? 2 : 1;
+    const int steps = ((int)(w->cols / QG) + 8 / wt - 1) / (8 / wt);
+    const size_t wgs = (pairs + wt - 1) / wt * ((m + 31) / 32), fit = PF_SK_PART_BYTES / (m * w->rows * 4);
+    const int want = (int)std::max<size_t>(1, std::min({(size_t)steps, (2 * ctx->cus + wgs - 1) / wgs, fit}));
+    const int each = (steps + want - 1) / want;
+    return (steps + each - 1) / each;
+}
+
 // The launch of a product of m tokens (epi, x, y and keys as qh_gemm takes them; `whole`: one partial).
 static Launch make_launch(const qh_ctx* ctx, const qh_mat* w, const void* x, size_t ldx, size_t m,
                           const int32_t* out_rows, void* y, int epi, uint64_t* keys, int whole, void* stream,
@@ -461,6 +476,7 @@ static Launch make_launch(const qh_ctx* ctx, const qh_mat* w, const void* x, siz
         l.waves = 4;
         l.tiles_per_wave = SKINNY_TILES;
         l.split = 1;  // the prefill launcher sets it (K-sliced plain products write several partials)
+        l.narrow = narrow_split(ctx, w, m, epi);
     }
     return l;
 }
@@ -533,6 +549,7 @@ int qh::gemm_with_scratch(qh_ctx* ctx, void* stream, const qh_mat* w, const void
         l.lora_split = lora->split;
         l.lora_cols = lora->m_cols;
         l.lora_rank = lora->rank;
+        if (l.narrow) l.narrow = 0, l.whole = 1;  // the prefill kernel, with as many partials
         l.lora_b = lora->b_f16;
         l.lora_tab = lora->tab;
         l.lora_tok_slot = lora->tok_slot;

@@ -39,6 +39,7 @@ struct Launch {
     int tiles_per_wave;     // skinny kernel: SKINNY_TILES, or 1 (plain int8 and bf16 products of 1-2 tokens)
     int nc;                 // skinny kernel: super-chunks of K (groups / (wave rows x groups_per_wave)); set at launch
     int mid;                // mid_kernel takes the product (9-48 tokens)
+    int narrow;             // more than 48 tokens, few bf16 rows: the splits of K on mid_kernel's blocks (0: prefill)
     int stage_out;          // skinny kernel, plain products: partials written through LDS in 16-byte row runs
     int cus;                // compute units (the prefill shape choice)
     int pf_shape;           // prefill workgroup shape: 0 chosen by size, else forced (kernels.hip prefill_epi)
@@ -100,6 +101,8 @@ constexpr int SKINNY_MAX_M = 48;
 // Split-K plain and SwiGLU products of 33-48 tokens on int4 and grouped int8 matrices of at least this many weights
 // take the prefill kernel (faster there; api.hip use_skinny).
 constexpr size_t PF_FROM33_WEIGHTS = (size_t)1 << 26;
+// Plain products of more tokens on dense bf16 matrices of up to this many tiles take mid_kernel (mid.h narrow_launch).
+constexpr int NARROW_TILES = 16;
 // 16-row tiles per wave in the skinny kernel, and its pipeline depth (groups whose loads are in flight + 1).
 #ifndef QH_SKINNY_TILES
 #define QH_SKINNY_TILES 2

@@ -2057,6 +2057,8 @@ static hipError_t prefill_epi(Launch& l) {
 template <int F, int EPI>
 hipError_t launch_epi(Launch& l) {
     if (l.skinny) return l.dry_run ? hipSuccess : skinny_epi<F & ~F_PERCH, EPI>(l);
+    if constexpr (F == F_BF16 && EPI == EPI_PLAIN)
+        if (l.narrow) return l.dry_run ? hipSuccess : narrow_launch<F>(l);
     return prefill_epi<F, EPI>(l);
 }
 template hipError_t launch_epi<QH_PART_F, QH_PART_EPI>(Launch& l);

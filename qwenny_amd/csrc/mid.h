@@ -59,7 +59,10 @@ static __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2)))
     const int wk = __builtin_amdgcn_readfirstlane(threadIdx.y), WK = blockDim.y;
     const int NW = WT * WK, wave = wk * WT + wt;
     const int l32 = lane & 31, lh = lane >> 5, l16 = lane & 15;
-    const int T = a.tiles, G = a.G, M = a.m;
+    const int T = a.tiles, G = a.G;
+    // the workgroup's tokens: all of them, or (narrow_launch) block blockIdx.z of 32 TB
+    const int M = min(a.m - 32 * TB * (int)blockIdx.z, 32 * TB);
+    const __bf16* const x0 = a.x + (size_t)(32 * TB) * blockIdx.z * a.ldx;
     const int tile0 = (blockIdx.x * WT + wt) * 2;
     const int tt = min(tile0 + (l32 >> 4), T - 1);
     const int s0 = blockIdx.y * a.spp, s1 = min(s0 + a.spp, a.steps);
@@ -82,7 +85,7 @@ static __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2)))
             const int g = min((s << a.gs_shift) + gi, G - 1);
             const int slot = 4 * q + (lane >> 4), row = min(slot, M - 1);
             const size_t xr = EPI == EPI_ARGMAX ? (size_t)xtab[row] : (size_t)row;
-            const __bf16* src = a.x + xr * a.ldx + (size_t)g * QG + 8 * ((lane & 15) ^ (slot & 15));
+            const __bf16* src = x0 + xr * a.ldx + (size_t)g * QG + 8 * ((lane & 15) ^ (slot & 15));
             __builtin_amdgcn_global_load_lds((const void*)src, (lds_ptr)(msmem + buf * XB + (gi * quads4 + q) * 1024), 16,
                                              0, 0);
         }
@@ -244,7 +247,7 @@ static __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2)))
                 ((__bf16*)a.y)[(size_t)tok * a.ldy + tile * 8 + l16] = (__bf16)(silu(val) * up);
         } else {
             if (tile_ok && tok < M)
-                __builtin_nontemporal_store(val, (float*)a.y + ((size_t)blockIdx.y * M + tok) * a.ldy + out);
+                __builtin_nontemporal_store(val, (float*)a.y + ((size_t)blockIdx.y * a.m + 32 * TB * blockIdx.z + tok) * a.ldy + out);
             if (EPI == EPI_ARGMAX) {
                 unsigned long long k = tile_ok && tok < M && out < a.valid ? argmax_key(val, out) : 0;
 #pragma unroll
@@ -323,4 +326,56 @@ static hipError_t mid_epi(const Launch& l) {
         return l.tile_waves == 2 ? mid_launch<F, EPI, TB, 2>(l) : hipErrorInvalidConfiguration;
     };
     return l.m > 32 ? go(std::integral_constant<int, 2>{}) : go(std::integral_constant<int, 1>{});
+}
+
+// y = the sum of `splits` partials of n4 float4 each, in order (y of any alignment)
+static __global__ __launch_bounds__(64) void sum_narrow_kernel(const float* x, int splits, size_t n4, float* y) {
+    const size_t i = (size_t)blockIdx.x * 64 + threadIdx.x;
+    if (i >= n4) return;
+    constexpr int B = 16;  // partials loaded ahead of their adds
+    f32x4 v = {0.0f, 0.0f, 0.0f, 0.0f};
+    for (int s0 = 0; s0 < splits; s0 += B) {
+        f32x4 p[B];
+#pragma unroll
+        for (int j = 0; j < B; j++)
+            if (s0 + j < splits) p[j] = ((const f32x4*)x)[(size_t)(s0 + j) * n4 + i];
+#pragma unroll
+        for (int j = 0; j < B; j++)
+            if (s0 + j < splits) v += p[j];
+    }
+#pragma unroll
+    for (int e = 0; e < 4; e++) y[4 * i + e] = v[e];
+}
+
+// Plain products of more than 48 tokens on dense bf16 matrices of few rows (up to NARROW_TILES tiles: a LoRA adapter's
+// stacked A, a DeltaNet in_ba projection), on mid_kernel over blocks of 32 tokens: the prefill kernel's 64 x 128 items
+// are a handful there, each walking all of K. Bound by the activations, read once; so K is split over the grid until
+// the launch has a few hundred workgroups, and a second launch (sum_narrow) adds the partials, kept in the stream-K
+// scratch, into one row of sums per token: split 1 to the caller (whose fused adapter epilogue then stages it in LDS).
+// Kernel trace at 333 tokens, 32 x 5120 / 16 x 17408: 29.7 us (24 items) -> 6.3 + 4.8 / 6.4 + 4.8 us (55 / 187
+// workgroups, then the sum).
+template <int F>
+static hipError_t narrow_launch(const Launch& l) {
+    static_assert(F == F_BF16, "dense bf16");
+    const int pairs = (l.rows / TILE + 1) / 2, wt = pairs >= 4 ? 4 : pairs >= 2 ? 2 : 1;
+    MidArgs a{};
+    a.codes = (const uint8_t*)l.codes;
+    a.x = (const __bf16*)l.x;
+    a.y = l.narrow > 1 ? (void*)l.sk_part : l.y;
+    a.ldx = l.ldx, a.ldy = l.ldy;
+    a.tiles = l.rows / TILE, a.G = l.cols / QG, a.m = l.m;
+    const int wk = 8 / wt;
+    a.gs_shift = wt == 4 ? 1 : wt == 2 ? 2 : 3;
+    a.steps = (a.G + wk - 1) / wk;
+    a.spp = (a.steps + l.narrow - 1) / l.narrow;
+    const size_t lds = std::max((size_t)mid_xbytes(32, a.gs_shift) * (a.spp > 1 ? 2 : 1), (size_t)8 * 4096);
+    const dim3 grid((pairs + wt - 1) / wt, l.narrow, (l.m + 31) / 32), block(64 * wt, wk);
+    if (wt == 4) hipLaunchKernelGGL((mid_kernel<F, EPI_PLAIN, 1, 4, false>), grid, block, lds, l.stream, a, NoLora{});
+    else if (wt == 2) hipLaunchKernelGGL((mid_kernel<F, EPI_PLAIN, 1, 2, false>), grid, block, lds, l.stream, a, NoLora{});
+    else hipLaunchKernelGGL((mid_kernel<F, EPI_PLAIN, 1, 1, false>), grid, block, lds, l.stream, a, NoLora{});
+    if (hipError_t e = hipGetLastError(); e != hipSuccess || l.narrow == 1) return e;
+    const size_t n4 = (size_t)l.m * l.rows / 4;
+    hipLaunchKernelGGL(sum_narrow_kernel, dim3((unsigned)((n4 + 63) / 64)), dim3(64), 0, l.stream, l.sk_part, l.narrow, n4,
+                       (float*)l.y);
+    return hipGetLastError();
 }
