@@ -287,12 +287,14 @@ struct Partition {
 // rows over K (each a group per step, two for int4) per workgroup, and the split of K over the grid (plain products
 // only, others need whole sums in one workgroup). Fitted to both kernels' times over 7 to 48 tokens, four formats and
 // 20 shapes (rows 1536-151936, K 1920-17408): 1.38x the speed of skinny_kernel in the geometric mean, 0.4% off the best
-// partition of each case. Sides measured, us (plain: with add_rmsnorm):
-// - plain int4: skinny_kernel's 4-group splits are ahead up to 16 tokens while their partials are few ((5120, 6144) at
-//   9 / 16 / 24 tokens 11.9 / 13.2 / 14.5 against 13.1 / 13.2 / 13.6; (5120, 17408) 21.7 / 24.8 / 30.7 against 20.2 /
-//   20.5 / 21.2), and above 32 tokens (17.9 against 19.5: two token blocks leave two waves per SIMD). Per-channel and
-//   grouped int8 up to 16 tokens likewise ((4096, 2560) at 9 10.6 against 10.8), but not on small matrices, and bf16
-//   (one group per skinny wave, a partial each) never.
+// partition of each case. Sides measured, us (plain: with add_rmsnorm, whose one launch takes few partials):
+// - plain: matrices of less than 320 tiles as pairs of tiles with eight wave rows, 2-5 partials, up to 16 tokens (wide
+//   formats 32, the LDS of their steps being half): (4096, 2560) at 9 / 16 tokens int4 10.9 / 11.7 -> 9.1 / 9.3, (9728,
+//   2560) bf16 20.7 / 22.3 -> 15.2 / 15.8; larger matrices and token counts with four or eight columns sharing the
+//   activations, 8-20 partials: (17408, 5120) int4 at 9 / 16 / 24 21.9 / 24.8 / 30.4 -> 19.9 / 20.8 / 21.1. skinny_kernel
+//   stays for int4 of 320 tiles and more up to 16 tokens while its 4-group splits are few ((6144, 5120) at 9 / 16 11.7 /
+//   12.9 against 12.9 / 13.6), and from 33 tokens but on small matrices (18.6 against 19.7: two token blocks leave two
+//   waves per SIMD).
 // - whole sums: skinny_kernel where its 16-tile workgroups of 8-16 waves fill the chip, from 2000 tiles (int4 up to 16
 //   tokens 27.6 against 29.9; argmax above 32 tokens); below that its few workgroups leave the chip idle (4096 x 2560
 //   whole rows 16-34 against 8-16).
@@ -303,15 +305,23 @@ static bool mid_partition(const qh_ctx* ctx, const qh_mat* m, size_t tokens, boo
     if (ctx->skinny_tile_waves || ctx->skinny_plain_wk != 1 || ctx->skinny_few) return false;
     const int T = (int)(m->rows / TILE), G = (int)(m->cols / QG), M = (int)tokens;
     const bool wide = is_i8(m->wt) || is_bf16(m->wt);  // formats of one group per wave and step
-    int wt, wk;
+    int wt, wk, aim = 0;  // aim: workgroups a plain launch aims for
     if (plain) {
-        const bool small = wide && (T <= 128 || (is_bf16(m->wt) && G < 32 && M <= 16));
-        if (!wide && (M > 32 || (M <= 16 && G < 96))) return false;
-        if (is_i8(m->wt) && M <= 16 && G < 64 && !small) return false;
-        wk = small ? 4 : 1;
-        if (small) wt = 1;
-        else if (!wide) wt = T >= 256 ? 8 : 4;
-        else wt = M > 32 || (T >= 256 && G < 32) ? 8 : 4;
+        if (!wide) {
+            if (M > 32 ? T > 160 || G >= 64 : M <= 16 && T >= 320 && G < 96) return false;
+            if (M <= 16 && T < 320) wt = 1, wk = 8, aim = 240;
+            else if (M <= 32 && T >= 320) wt = 8, wk = 1, aim = 240;
+            else if (M <= 32 && T <= 128) wt = 1, wk = 4, aim = 256;
+            else wt = 4, wk = 1, aim = G >= 64 ? 384 : 256;
+        } else if (M > 32) {
+            if (T <= 128) wt = 1, wk = 4, aim = 256;
+            else if (T < 320) wt = 4, wk = 1, aim = G >= 64 ? 384 : 256;
+            else wt = 8, wk = 1, aim = 240;
+        } else if (T < 320) {
+            wt = 1, wk = 8, aim = M <= 16 ? 256 : 240;
+        } else {
+            wt = G <= 64 ? 1 : 4, wk = G <= 64 ? 4 : 1, aim = 480;
+        }
     } else if (wide) {
         if (M > 32 && argmax) return false;
         if (T <= 512) wt = 1, wk = M > 32 ? 4 : 8;
@@ -327,10 +337,10 @@ static bool mid_partition(const qh_ctx* ctx, const qh_mat* m, size_t tokens, boo
     }
     int split = 1;
     if (plain) {
-        // workgroups the launch aims for: about 1000-1900 waves
-        const int aim = wt == 1 ? 384 : wt == 8 ? 240 : wide ? 384 : 256;
         const int per = wk * (wide ? 1 : 2), steps = (G + per - 1) / per, columns = (T + 2 * wt - 1) / (2 * wt);
-        const int want = std::max(1, std::min(steps, (aim + columns - 1) / columns));
+        // (eight wave rows: two steps per split where there are more than three)
+        const int most = wk == 8 && steps > 3 ? std::max(2, (steps + 1) / 2) : steps;
+        const int want = std::max(1, std::min(most, (aim + columns - 1) / columns));
         const int each = (steps + want - 1) / want;  // steps per split
         split = (steps + each - 1) / each;
     }

@@ -43,10 +43,8 @@ __global__ __launch_bounds__(256) void sum_parts_kernel(const float4* __restrict
     }
 }
 
-constexpr int AR_THREADS = 256;
-// add_rmsnorm spreads the partials' sum over workgroups below this many float4 per step (n * hidden / 4): 64 tokens
-// of a 5120-wide row, where a workgroup per token leaves most CUs idle
-constexpr long AR_SPREAD_BELOW = 64l * 1280;
+// add_rmsnorm takes one launch up to this many floats of partials per row (a row is one workgroup's, about 100 GB/s)
+constexpr size_t AR_ROW_FLOATS = 40960;
 
 // y[t] = bf16(w * (h[t] / rms(h[t]))) with the row held in registers: each of the T threads loads its C float4 of h
 // and of w at once (one memory round trip), then the sum of squares and the output (H4 <= T * C)
@@ -82,6 +80,70 @@ __global__ __launch_bounds__(T) void rmsnorm_kernel(const float* __restrict__ h,
         yo[1] = (__bf16)(wn[i].y * (v[i].y * r));
         yo[2] = (__bf16)(wn[i].z * (v[i].z * r));
         yo[3] = (__bf16)(wn[i].w * (v[i].w * r));
+    }
+}
+
+// The whole step in one launch, a workgroup per token with the row in registers: each thread takes C float4 of the row
+// (every blockDim.x-th), loads its h, w and B partials of each at once, adds the partials in order, writes h, and
+// normalises once the workgroup's sum of squares is known.
+template <int C, int B>
+__global__ __launch_bounds__(1024) void row_norm_kernel(float* __restrict__ h, const float* __restrict__ x, int splits,
+                                                        int n, int H, const float* __restrict__ w,
+                                                        __bf16* __restrict__ y, float eps) {
+    __shared__ float wsum[16];
+    const int T = blockDim.x, H4 = H / 4;
+    float4* const hr = (float4*)(h + (size_t)blockIdx.x * H);
+    const float4* const xr = (const float4*)x + (size_t)blockIdx.x * H4;
+    const size_t n4 = (size_t)n * H4;
+    float4 v[C], wn[C];
+    float ss = 0.0f;
+#pragma unroll
+    for (int i = 0; i < C; i++) {
+        const int c = threadIdx.x + i * T;
+        v[i] = c < H4 ? hr[c] : make_float4(0.0f, 0.0f, 0.0f, 0.0f);
+    }
+    for (int s0 = 0; s0 < splits; s0 += B) {
+        float4 p[C][B];
+#pragma unroll
+        for (int i = 0; i < C; i++) {
+            const int c = threadIdx.x + i * T;
+#pragma unroll
+            for (int j = 0; j < B; j++)
+                p[i][j] = c < H4 && s0 + j < splits ? xr[(size_t)(s0 + j) * n4 + c] : make_float4(0.0f, 0.0f, 0.0f, 0.0f);
+        }
+        if (s0 == 0) {
+#pragma unroll
+            for (int i = 0; i < C; i++) {
+                const int c = threadIdx.x + i * T;
+                wn[i] = c < H4 ? ((const float4*)w)[c] : make_float4(0.0f, 0.0f, 0.0f, 0.0f);
+            }
+        }
+#pragma unroll
+        for (int i = 0; i < C; i++)
+#pragma unroll
+            for (int j = 0; j < B; j++)
+                if (s0 + j < splits) v[i].x += p[i][j].x, v[i].y += p[i][j].y, v[i].z += p[i][j].z, v[i].w += p[i][j].w;
+    }
+#pragma unroll
+    for (int i = 0; i < C; i++) {
+        const int c = threadIdx.x + i * T;
+        if (c < H4) hr[c] = v[i];
+        ss += v[i].x * v[i].x + v[i].y * v[i].y + v[i].z * v[i].z + v[i].w * v[i].w;
+    }
+    for (int o = 32; o > 0; o >>= 1) ss += __shfl_xor(ss, o);
+    if ((threadIdx.x & 63) == 0) wsum[threadIdx.x >> 6] = ss;
+    __syncthreads();
+    float tot = 0.0f;
+    for (int i = 0; i < T / 64; i++) tot += wsum[i];
+    const float r = rsqrtf(tot / (float)H + eps);
+#pragma unroll
+    for (int i = 0; i < C; i++) {
+        const int c = threadIdx.x + i * T;
+        if (c >= H4) break;
+        typedef __bf16 b4 __attribute__((ext_vector_type(4)));
+        const b4 o = {(__bf16)(wn[i].x * (v[i].x * r)), (__bf16)(wn[i].y * (v[i].y * r)),
+                      (__bf16)(wn[i].z * (v[i].z * r)), (__bf16)(wn[i].w * (v[i].w * r))};
+        __builtin_memcpy(y + (size_t)blockIdx.x * H + 4 * c, &o, 8);
     }
 }
 
@@ -467,20 +529,50 @@ extern "C" int qh_add_rmsnorm(void* stream, float* h, const float* x, int splits
     if (hidden == 0 || hidden % 4 || hidden > (1u << 24) || n > 0x7fffffffu || (uintptr_t)h % 16 ||
         (uintptr_t)x % 16 || (uintptr_t)w_next % 16)
         return fail(QH_EINVAL, "add_rmsnorm: hidden %zu must be a multiple of 4, f32 buffers 16-byte aligned", hidden);
-    // few tokens (decode): the partials' sum, the bulk of the bytes, over many workgroups first (a workgroup per token
-    // would read a 34-split partial set of a 5120-wide row alone, about 20 us), then the norm with no partials left
-    const long n4 = (long)(n * hidden / 4);
-    if (splits > 1 && (long)n * (hidden / 4) < (long)AR_SPREAD_BELOW) {
-        if (sum_launch((hipStream_t)stream, x, splits, n4, nullptr, h)) return fail(QH_EHIP, "add_rmsnorm launch failed");
+    // One launch with the row in registers (row_norm_kernel) unless a row has more partials than its workgroup loads at
+    // once (16, and AR_ROW_FLOATS in all) and the tokens are up to 64 (few workgroups): then the partials' sum over many
+    // workgroups first, the norm afterwards. Graph replays after a kernel that writes the partials, us, two launches
+    // against one: 5120 wide, 1 token, 1 / 4 / 8 / 12 partials 4.6 / 4.1 / 4.3 / 4.2 against 2.4 / 3.3 / 4.3 / 5.8, 20
+    // tokens 5.3 / 5.0 / 5.7 / 6.4 against 2.9 / 4.1 / 5.6 / 7.6; 2560 wide, 1 token, 4 / 12 / 16 / 19 3.8 / 3.8 / 3.9 /
+    // 4.2 against 2.3 / 3.4 / 3.7 / 4.5, 48 tokens 4.8 / 6.8 / 7.4 / 6.8 against 3.4 / 5.9 / 6.3 / 6.7; 5120 wide, 100
+    // tokens, 8 partials 9.2 against 7.4. Streaming sizes, against a workgroup of 256 threads that reads its row again to
+    // normalise it: 5120 wide, 333 tokens, 1 / 4 partials 8.7 / 10.5 -> 6.6 / 9.4, 2048 tokens 29.9 / 57.0 -> 24.7 / 54.5.
+    const size_t H4 = hidden / 4;
+    const bool stream_rows = n > 256;
+    if (H4 <= 1024 * 4 && (n > 64 || (splits <= 16 && (size_t)splits * hidden <= AR_ROW_FLOATS))) {
+        // float4 per thread and partials loaded ahead: one column each where a workgroup holds them (the shortest chain),
+        // two, or four, and one partial at a time, at streaming sizes (more rows in flight per CU)
+        const int c = H4 > 2048 || n >= 1024 ? 4 : H4 > 1024 || stream_rows ? 2 : 1;
+        const unsigned t = (unsigned)(((H4 + c - 1) / c + 63) / 64 * 64);
+        auto go = [&](auto Cc, auto Bc) {
+            hipLaunchKernelGGL((row_norm_kernel<decltype(Cc)::value, decltype(Bc)::value>), dim3((unsigned)n), dim3(t), 0,
+                               (hipStream_t)stream, h, x, splits, (int)n, (int)hidden, w_next, (__bf16*)y_bf16, eps);
+        };
+        using I1 = std::integral_constant<int, 1>;
+        using I2 = std::integral_constant<int, 2>;
+        using I4 = std::integral_constant<int, 4>;
+        using I8 = std::integral_constant<int, 8>;
+        using I16 = std::integral_constant<int, 16>;
+        if (c == 4) go(I4{}, I1{});
+        else if (c == 2) {
+            if (stream_rows || splits <= 2) go(I2{}, I1{});
+            else if (splits <= 4) go(I2{}, I4{});
+            else go(I2{}, I8{});
+        } else if (splits <= 4) go(I1{}, I4{});
+        else if (splits <= 8 || n > 64) go(I1{}, I8{});
+        else go(I1{}, I16{});
+    } else if (splits > 1 && n <= 64) {
+        if (sum_launch((hipStream_t)stream, x, splits, (long)(n * H4), nullptr, h))
+            return fail(QH_EHIP, "add_rmsnorm launch failed");
         // the norm alone, a wide workgroup per token with the row in registers
-        if (hidden / 4 <= 1024 * 4)
+        if (H4 <= 1024 * 4)
             hipLaunchKernelGGL((rmsnorm_kernel<1024, 4>), dim3((unsigned)n), dim3(1024), 0, (hipStream_t)stream, h,
                                (int)hidden, w_next, (__bf16*)y_bf16, eps);
         else
             hipLaunchKernelGGL(add_rmsnorm_kernel<1024>, dim3((unsigned)n), dim3(1024), 0, (hipStream_t)stream, h, x,
                                0, (int)n, (int)hidden, w_next, (__bf16*)y_bf16, eps);
     } else {
-        hipLaunchKernelGGL(add_rmsnorm_kernel<AR_THREADS>, dim3((unsigned)n), dim3(AR_THREADS), 0, (hipStream_t)stream,
+        hipLaunchKernelGGL(add_rmsnorm_kernel<256>, dim3((unsigned)n), dim3(256), 0, (hipStream_t)stream,
                            h, x, splits, (int)n, (int)hidden, w_next, (__bf16*)y_bf16, eps);
     }
     if (hipError_t e = hipGetLastError(); e != hipSuccess)

@@ -1,0 +1,34 @@
+"""add_rmsnorm on both of its paths (one launch with the row in registers, or the partials' sum first): rows of one to
+four float4 per thread and a remainder, partials of every batch size, decode and streaming token counts, at the bound
+between the paths. The residual is bit-exact against the oracle's order, the bf16 output within one bf16 rounding of the
+f64 norm."""
+
+import numpy as np
+import pytest
+
+import oracle
+from qwenny_amd import add_rmsnorm
+from tests.helpers import bf16_out_err
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.mark.parametrize("splits,n,hidden", [(1, 1, 4), (2, 3, 20), (3, 2, 1152), (4, 65, 2560), (5, 3, 5120), (9, 2, 5120),
+                                             (10, 2, 5120), (12, 5, 4096), (13, 5, 4096), (17, 2, 1152), (19, 1, 2560),
+                                             (20, 64, 2560), (8, 100, 5120), (2, 300, 2560), (1, 1030, 1024),
+                                             (2, 3, 16384), (1, 257, 8200), (3, 2, 16388)])
+def test_add_rmsnorm_paths(splits, n, hidden):
+    import torch
+
+    print(f"row norm {splits}x{n}x{hidden}", flush=True)
+    rng = np.random.default_rng(hidden + splits + n)
+    h = rng.standard_normal((n, hidden)).astype(np.float32)
+    x = (rng.standard_normal((splits, n, hidden)) * 0.3).astype(np.float32)
+    w = rng.uniform(0.5, 1.5, hidden).astype(np.float32)
+    hd, xd, wd = (torch.from_numpy(a).cuda() for a in (h, x, w))
+    y = torch.full((n, hidden), float("nan"), dtype=torch.bfloat16, device="cuda")
+    add_rmsnorm(None, hd, xd, splits, n, hidden, wd, y, 1e-6)
+    torch.cuda.synchronize()
+    want_h, want_y = oracle.add_rmsnorm(h, x, splits, w, 1e-6)
+    assert np.array_equal(hd.cpu().numpy(), want_h)
+    assert bf16_out_err(y.float().cpu().numpy(), want_y) <= 1e-5
