@@ -281,6 +281,7 @@ extern "C" int qh_mat_download(const qh_mat* m, void* codes, void* scales, void*
 struct Partition {
     int tile_waves, waves, split, groups_per_wave, tiles_per_wave;
     bool mid = false;  // mid_kernel takes the product
+    bool mw = false;   // skinny_mw_kernel does (plain, split)
 };
 
 // mid_kernel's partition of a product of 9-48 tokens, false where skinny_kernel stays: wave columns of two tiles x wave
@@ -348,6 +349,27 @@ static bool mid_partition(const qh_ctx* ctx, const qh_mat* m, size_t tokens, boo
     return true;
 }
 
+// skinny_mw_kernel's partition of a plain product of 1-8 tokens: two or three splits of K, few partials, the rest of K
+// over the workgroup's waves. A consumer's sum of the partials costs by their number (add_rmsnorm takes one launch up to
+// 16, fewer of wide rows), and small matrices leave skinny_kernel few waves per CU unless it writes a partial per group.
+// Taken by wide formats up to 384 tiles and by int4 up to 319 tiles from 2 tokens. Same-box graph replays, us with
+// add_rmsnorm (alone), skinny_kernel and its lean forms against this, at 1 / 4 / 8 tokens: (4096, 2560) int4 - / 10.6
+// (4.7) / 11.6 (5.3) -> - / 7.9 (4.9) / 8.2 (5.0), int8 9.7 (4.4) / 11.2 (5.3) / 11.5 (5.5) -> 8.5 (5.4) / 8.6 (5.5) / 8.9
+// (5.8); (9728, 2560) int4 - / 10.9 (5.2) / 11.4 (5.5) -> - / 9.6 (6.0) / 9.9 (6.2), bf16 17.4 (9.6) / 19.6 (10.9) / 20.1
+// (11.5) -> 13.3 (9.8) / 13.5 (9.9) / 13.8 (10.3); (17408, 5120) int8 23.1 (16.8) / 25.9 (19.1) / 26.3 (19.4) -> 21.7
+// (17.4) / 22.0 (17.6) / 23.1 (18.5). One-token int4 and int4 of 320 tiles and more keep their lean kernels, whose
+// products alone are faster ((17408, 5120) at 5 tokens 17.7 (10.8) against 16.3 (11.9)).
+static bool mw_partition(const qh_ctx* ctx, const qh_mat* m, size_t tokens, Partition* out) {
+    if (tokens < 1 || tokens > 8 || ctx->skinny_tile_waves || ctx->skinny_plain_wk != 1 || ctx->skinny_few) return false;
+    const int T = (int)(m->rows / TILE), G = (int)(m->cols / QG);
+    const bool wide = is_i8(m->wt) || is_bf16(m->wt);
+    if (wide ? T > 384 : T >= 320 || tokens == 1) return false;
+    const int ng = is_bf16(m->wt) ? 1 : is_i8(m->wt) ? 2 : 4;  // groups per wave (mw_ng)
+    const int chunks = (G + ng - 1) / ng, want = std::min(chunks, G >= 48 ? 3 : 2), each = (chunks + want - 1) / want;
+    *out = Partition{1, std::min(8, each), (chunks + each - 1) / each, ng, SKINNY_TILES, false, true};
+    return true;
+}
+
 // The skinny kernel's partition of a product of m tokens (kernels.hip skinny_kernel): each wave takes SKINNY_TILES
 // tiles (plain int8 and bf16 products of 1-2 tokens: one) and 4 groups (1 when the group count is not a multiple of 4); a
 // workgroup stages the activations of its super-chunk of K once for all its waves, so the more wave columns
@@ -360,6 +382,7 @@ static bool mid_partition(const qh_ctx* ctx, const qh_mat* m, size_t tokens, boo
 static Partition skinny_partition(const qh_ctx* ctx, const qh_mat* m, size_t tokens, bool plain,
                                   bool argmax = false) {
     if (Partition p; mid_partition(ctx, m, tokens, plain, argmax, &p)) return p;
+    if (Partition p; plain && mw_partition(ctx, m, tokens, &p)) return p;
     const int tiles = (int)(m->rows / TILE), G = (int)(m->cols / QG);
     // tiles per wave: one for plain int8 and bf16 products of 1-2 tokens (8 KiB of one tile, half the registers of a
     // two-tile wave, 5 waves per SIMD for int8: same-box graph replays, int8 per channel 27B set at M = 1 5.39 -> 5.49
@@ -473,6 +496,7 @@ static Launch make_launch(const qh_ctx* ctx, const qh_mat* w, const void* x, siz
     if (l.skinny) {
         Partition p = skinny_partition(ctx, w, m, epi == QH_EPI_PLAIN && !whole, epi == QH_EPI_ARGMAX);
         l.mid = p.mid;
+        l.mw = p.mw;
         l.tile_waves = p.tile_waves;
         l.waves = p.waves;
         l.split = p.split;

@@ -39,6 +39,7 @@ struct Launch {
     int tiles_per_wave;     // skinny kernel: SKINNY_TILES, or 1 (plain int8 and bf16 products of 1-2 tokens)
     int nc;                 // skinny kernel: super-chunks of K (groups / (wave rows x groups_per_wave)); set at launch
     int mid;                // mid_kernel takes the product (9-48 tokens)
+    int mw;                 // skinny_mw_kernel takes the (plain, split) product
     int narrow;             // more than 48 tokens, few bf16 rows: the splits of K on mid_kernel's blocks (0: prefill)
     int stage_out;          // skinny kernel, plain products: partials written through LDS in 16-byte row runs
     int cus;                // compute units (the prefill shape choice)

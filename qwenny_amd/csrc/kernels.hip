@@ -1032,7 +1032,8 @@ static __global__ __launch_bounds__(512) void skinny_mt_kernel(MtArgs a) {
 // epilogue), with or without an adapter: skinny_m1w_kernel's partition (a workgroup per tile pair over all of K, each
 // wave taking every WK-th chunk of NG groups, 8 KiB of codes in flight) with skinny_mt_kernel's token rows (each wave
 // stages its tokens' rows of its chunk, 16 bytes apart; token 4 r + lane / 16 in row r of a lane's accumulators). The
-// waves' sums meet in LDS and are added in wave order. A last chunk of fewer than NG groups reads its last group again.
+// waves' sums meet in LDS and are added in wave order. Plain products of small matrices run on it too, K cut into a few
+// splits over the grid (api.hip mw_partition). A last chunk of fewer than NG groups reads its last group again.
 // HBM-bound, and latency-bound in skinny_kernel, whose workgroups of 2-8 wave columns are few on matrices of this size
 // and walk K one staged super-chunk after another.
 struct MwArgs {
@@ -1043,6 +1044,7 @@ struct MwArgs {
     int ldx;
     void* y;  // plain: f32 [m][tiles * 16]; SwiGLU: bf16 [m][tiles * 8]
     int tiles, G, m;
+    int gps;  // groups of K per split (blockIdx.y), a multiple of NG; all of them for whole sums
     uint32_t mask, magic;
 };
 struct NoLora {};
@@ -1074,7 +1076,8 @@ static __global__ __launch_bounds__(512) void skinny_mw_kernel(MwArgs a, std::co
         for (int r = 0; r < NR; r++) acc[t][r] = 0.0f;
     // MFMA row l16 holds token 4 (l16 % 4) + l16 / 4; rows past M read row M - 1 (never stored)
     const __bf16* xrow0 = xw + min(((l16 & 3) << 2) | (l16 >> 2), M - 1) * XP + 8 * kq;
-    for (int gw = NG * wk; gw < G; gw += NG * WK) {
+    const int g1 = min((int)(blockIdx.y + 1) * a.gps, G);
+    for (int gw = blockIdx.y * a.gps + NG * wk; gw < g1; gw += NG * WK) {
         const int col = min(gw * QG + 8 * lane, G * QG - 8);
         for (int r = 0; r < M; r++)
             if (NG == 4 || lane < 16 * NG)
@@ -1152,7 +1155,7 @@ static __global__ __launch_bounds__(512) void skinny_mw_kernel(MwArgs a, std::co
         }
     }
     if constexpr (LORA) {
-        if (wk == 0) {
+        if (wk == 0 && blockIdx.y == 0) {
 #pragma unroll
             for (int t = 0; t < 2; t++) {
                 if (tile0 + t >= T) break;
@@ -1183,7 +1186,8 @@ static __global__ __launch_bounds__(512) void skinny_mw_kernel(MwArgs a, std::co
             if (tile < T && !(row & 8))
                 ((__bf16*)a.y)[(size_t)tok * T * (TILE / 2) + tile * (TILE / 2) + (row & 7)] = (__bf16)(silu(v) * up);
         } else if (tile < T) {
-            __builtin_nontemporal_store(v, (float*)a.y + (size_t)tok * T * TILE + tile * TILE + (row & 15));
+            __builtin_nontemporal_store(
+                v, (float*)a.y + ((size_t)blockIdx.y * M + tok) * T * TILE + tile * TILE + (row & 15));
         }
     }
 }
@@ -1191,11 +1195,11 @@ static __global__ __launch_bounds__(512) void skinny_mw_kernel(MwArgs a, std::co
 template <int F, int EPI>
 static hipError_t mw_launch(const Launch& l, int wk) {
     constexpr int NG = mw_ng<F>();
-    const int tiles = l.rows / TILE;
-    const MwArgs a{(const u32x4*)l.codes, l.scales, l.zeros, (const __bf16*)l.x, l.ldx, l.y, tiles, l.cols / QG, l.m,
+    const int tiles = l.rows / TILE, G = l.cols / QG, nc = (G + NG - 1) / NG, gps = (nc + l.split - 1) / l.split * NG;
+    const MwArgs a{(const u32x4*)l.codes, l.scales, l.zeros, (const __bf16*)l.x, l.ldx, l.y, tiles, G, l.m, gps,
                    l.nib_mask, l.bf16_magic};
     const size_t lds = (size_t)wk * l.m * mt_xpitch<NG>() * 2 + (size_t)wk * l.m * 32 * 4;
-    const dim3 grid((tiles + 1) / 2), block(64 * wk);
+    const dim3 grid((tiles + 1) / 2, l.split), block(64 * wk);
     auto go = [&](auto NRc) {
         constexpr int NR = decltype(NRc)::value;
         if (l.lora_rank) hipLaunchKernelGGL((skinny_mw_kernel<F, EPI, NR, true>), grid, block, lds, l.stream, a, l);
@@ -1849,6 +1853,7 @@ static hipError_t skinny_epi(const Launch& l) {
         // 11.6 / 12.1 / 12.7. Beyond 8 tokens against mid_kernel, at 9 / 12 / 16: 4864 x 2432 int4 7.2 / 7.8 / 8.0 ->
         // 5.6 / 6.1 / 5.9, 19456 x 2560 13.1 / 13.0 / 13.2 -> 9.6 / 11.9 / 15.0, 34816 x 5120 27.6 / 28.7 / 29.0 ->
         // 33.5 / 33.5 / 32.1 (its activations staged by every wave), int8 44.3 / 39.7 / 41.1 -> 34.7 / 36.8 / 46.0.
+        if (l.mw) return mw_launch<F, EPI>(l, l.waves);
         const int tiles = l.rows / TILE;
         const int most = tiles <= 512 ? 16 : tiles <= 1536 || (F & F_I8) ? 12 : 8;
         if (l.m <= most && (EPI == EPI_SILU || l.whole) && !l.xrows)

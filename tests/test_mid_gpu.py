@@ -1,5 +1,5 @@
 """Products of 9-48 tokens on mid_kernel (whose partition depends on the matrix's tiles, groups and storage, and on the
-token count) and whole sums of 1-16 tokens on skinny_mw_kernel: odd tile counts and group counts, one tile, one group, both token blocks and their last rows, every
+token count) and whole sums of 1-16 tokens and few-split products of 1-8 on skinny_mw_kernel: odd tile counts and group counts, one tile, one group, both token blocks and their last rows, every
 storage and epilogue, gathered logit rows. Products are exact products of the dequantized weights, so the bar is the
 decode kernels' 1e-4 against the f64 oracle (measured 1e-6: f32 sums of up to 2432 terms), one bf16 ulp beyond it for
 SwiGLU outputs."""
@@ -27,7 +27,7 @@ def _matrix(gemm, kind, n, k, silu=False):
 
 
 SHAPES = [(16, 128), (48, 2432), (528, 384), (2064, 1280), (4112, 640), (8208, 256), (24592, 128), (32800, 128),
-          (336, 12672)]
+          (336, 12672), (2560, 6272)]
 
 
 @pytest.mark.parametrize("kind", ["i4", "i4z", "i4s32", "i8", "i8g", "bf16"])
@@ -36,7 +36,7 @@ def test_plain_and_whole(gemm, kind, n, k):
     import torch
 
     mat, want_of = _matrix(gemm, kind, n, k)
-    for m in (1, 4, 5, 8, 9, 13, 16, 17, 25, 32, 33, 48):
+    for m in (1, 2, 4, 5, 8, 9, 13, 16, 17, 25, 32, 33, 48):
         x = activations(m, "x", m, k)
         want = want_of(x)
         split = mat.split(m)
