@@ -266,15 +266,81 @@ __device__ void lora_delta16(const Launch& a, int tile, int tok0, f32x4& d) {
     }
 }
 
+// The same delta of a tile pair for kernels whose waves' accumulators are summed afterwards, from LDS: each wave takes a
+// share of the steps of every module of tiles tile0, tile0 + 1, two at a time, into d[tile]. The pair's B rows and the
+// tokens' xa partials are staged when the kernel starts (lora_stage16, 4 bytes per lane global -> LDS, ahead of the
+// weights), the module table read there too, so that no chain of loads follows the last chunk. Kernel trace, us, against
+// one wave reading them from memory at the end: 27B [gate; up], rank 16, one token 25.5 -> 23.2; 4B with zero points, rank
+// 64, 5 tokens, [gate; up] 18.7 -> 16.2, down 12.8 -> 11.1. (At one token and for int8 the kernel is held to six waves per
+// SIMD, as without adapter: 26.3 us at five.)
+struct Lora16 {
+    const float* xa;     // [split][m][cols]
+    const _Float16* b;   // the tile pair's rows: [32][rank]
+    int end[3], off[4];  // the modules' end rows and first columns of xa
+};
+__host__ __device__ inline int lora16_bytes(int split, int m, int cols, int rank) {
+    return ((split * m * cols * 4 + 255) & ~255) + 32 * rank * 2;
+}
+// LDS a decode launch gives to it at most
+constexpr int LORA16_MAX = 24 * 1024;
+
+__device__ __forceinline__ Lora16 lora_stage16(const Launch& a, int tile0, uint8_t* lds, int wave, int waves) {
+    const int lane = threadIdx.x & 63, nx = a.lora_split * a.m * a.lora_cols, bx = (nx * 4 + 255) & ~255;
+    auto copy = [&](const uint32_t* src, int n, uint8_t* dst) __attribute__((always_inline)) {  // n words
+        for (int i = wave * 64; i < n; i += waves * 64)  // (past the end: the last word again, into the padding)
+            __builtin_amdgcn_global_load_lds((const void*)(src + min(i + lane, n - 1)),
+                                             (__attribute__((address_space(3))) void*)(dst + i * 4), 4, 0, 0);
+    };
+    copy((const uint32_t*)a.lora_xa, nx, lds);
+    // the last pair of an odd tile count: its second tile's rows are clamped away (never used)
+    const int rows = min(32, a.rows - tile0 * TILE);
+    copy((const uint32_t*)(a.lora_b + (size_t)tile0 * TILE * a.lora_rank), rows * a.lora_rank / 2, lds + bx);
+    const int* const tab = a.lora_tab;
+    return Lora16{(const float*)lds, (const _Float16*)(lds + bx), {tab[0], tab[1], tab[2]}, {tab[4], tab[5], tab[6], tab[7]}};
+}
+
+template <bool SILU>
+__device__ void lora_share16(const Launch& a, const Lora16& st, float s, int tile0, int tiles, int share, int nshare,
+                             f32x4 (&d)[2]) {
+    constexpr int C = 2;
+    const int Q = a.lora_rank / 4;
+    const int lane = threadIdx.x & 63, l16 = lane & 15, q = lane >> 4;
+    const int tok = min(((l16 & 3) << 2) | (l16 >> 2), a.m - 1);
+    int n = 0;  // pairs of steps passed
+#pragma unroll
+    for (int t = 0; t < 2; t++) {
+        const int tile = tile0 + t, o = tile * TILE + l16;
+        if (tile >= tiles) break;  // wave-uniform
+        auto module = [&](int r) { return SILU ? (r >> 3) & 1 : (r >= st.end[0]) + (r >= st.end[1]) + (r >= st.end[2]); };
+        const int mod = module(o), mlo = module(tile * TILE), mhi = module(tile * TILE + TILE - 1);
+        for (int m = mlo; m <= mhi; m++) {
+            const int c0 = m < 2 ? (m ? st.off[1] : st.off[0]) : (m == 2 ? st.off[2] : st.off[3]);
+            if (c0 < 0) continue;  // wave-uniform
+            for (int i0 = 0; i0 < Q; i0 += C, n++) {
+                if (n % nshare != share) continue;
+                float xv[C] = {0.0f, 0.0f};
+                for (int sp = 0; sp < a.lora_split; sp++)
+#pragma unroll
+                    for (int i = 0; i < C; i++) xv[i] += st.xa[(sp * a.m + tok) * a.lora_cols + c0 + q * Q + i0 + i];
+                const _Float16* bp = st.b + (t * TILE + l16) * a.lora_rank + q * Q + i0;
+#pragma unroll
+                for (int i = 0; i < C; i++)
+                    d[t] = __builtin_amdgcn_mfma_f32_16x16x4f32(xv[i] * s, mod == m ? (float)bp[i] : 0.0f, d[t], 0, 0, 0);
+            }
+        }
+    }
+}
+
 // The prefill kernel's layout (v_mfma_f32_32x32x2_f32): the deltas of a wave's TN blocks of 32 output rows (block t:
 // rows (tile0 + 2 t) 16 ..) for its BMB blocks of 32 tokens (block bb: tokens tok0 + 32 bb ..), accumulated into
 // acc[bb][t]; lane l holds D[token 8 (v / 4) + 4 (l / 32) + v % 4][row l % 32], v = 0..15. Loads are batched for
 // latency: the tokens' slot scales for every block at once, each lane's B run once, and xa either from the item's rows
 // staged in LDS (xs: one split, 4-32 columns; row r's 16-byte chunk k at slot k ^ (r mod chunks per row), rows from
-// xs_row0) or, otherwise, the xa runs of NBB token blocks at a time from global memory.
+// xs_row0) or, otherwise, the xa runs of NBB token blocks at a time from global memory. share of nshare: every
+// nshare-th batch of steps (waves whose accumulators are summed afterwards).
 template <bool SILU, int BMB, int TN>
 __device__ void lora_item32(const Launch& a, int tile0, int tok0, f32x16 (&acc)[BMB][TN], const uint8_t* xs = nullptr,
-                            int xs_row0 = 0) {
+                            int xs_row0 = 0, int share = 0, int nshare = 1) {
     // one code path for every rank (a switch over ranks multiplies the epilogue's code and spills registers): the
     // H = R / 2 contraction steps run C at a time, lane group h taking k = h H + i
     constexpr int C = 4;                     // steps whose operands are in registers at a time (H is a multiple)
@@ -315,7 +381,7 @@ __device__ void lora_item32(const Launch& a, int tile0, int tok0, f32x16 (&acc)[
         for (int m = mlo; m <= mhi; m++) {
             const int c0 = lora_off(a, m);
             if (c0 < 0) continue;  // wave-uniform
-            for (int i0 = 0; i0 < H; i0 += C) {
+            for (int i0 = C * share; i0 < H; i0 += C * nshare) {
                 float bv[C];
                 const bool keep = mod == m && o0 + l32 < a.rows;
 #pragma unroll
@@ -1045,6 +1111,7 @@ struct MwArgs {
     void* y;  // plain: f32 [m][tiles * 16]; SwiGLU: bf16 [m][tiles * 8]
     int tiles, G, m;
     int gps;  // groups of K per split (blockIdx.y), a multiple of NG; all of them for whole sums
+    int lora_staged;  // an adapter's B rows and xa staged in LDS (else read from memory after the last chunk)
     uint32_t mask, magic;
 };
 struct NoLora {};
@@ -1054,7 +1121,9 @@ template <int F>
 __host__ __device__ constexpr int mw_ng() { return 4 / CodeWords<F>::N; }
 
 template <int F, int EPI, int NR, bool LORA>
-static __global__ __launch_bounds__(512) void skinny_mw_kernel(MwArgs a, std::conditional_t<LORA, Launch, NoLora> ll) {
+static __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(
+    LORA && ((F == F_I4 && NR == 1) || (F & F_I8)) ? 6 : 2))) void skinny_mw_kernel(
+    MwArgs a, std::conditional_t<LORA, Launch, NoLora> ll) {
     extern __shared__ __attribute__((aligned(16))) uint8_t smem[];
     constexpr int NG = mw_ng<F>(), XP = mt_xpitch<NG>(), CW = CodeWords<F>::N;
     const int lane = threadIdx.x & 63, wk = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
@@ -1068,6 +1137,15 @@ static __global__ __launch_bounds__(512) void skinny_mw_kernel(MwArgs a, std::co
     asm volatile("v_mov_b32 %0, %1" : "=v"(magic) : "s"(a.magic));
     const uint32_t mask = a.mask;
     const int tl[2] = {tile0, t1};
+    Lora16 lst{};
+    int slot = 0;      // the lane's token's adapter slot, then its scale
+    float lscale = 0.0f;
+    if constexpr (LORA) {
+        if (blockIdx.y == 0 && a.lora_staged) {
+            slot = ll.lora_tok_slot[min(((l16 & 3) << 2) | (l16 >> 2), M - 1)];
+            lst = lora_stage16(ll, tile0, (uint8_t*)(red + (size_t)WK * M * 32), wk, WK);
+        }
+    }
     const bf16x8 ones = __builtin_bit_cast(bf16x8, u32x4{0x3F803F80u, 0x3F803F80u, 0x3F803F80u, 0x3F803F80u});
     float acc[2][NR];
 #pragma unroll
@@ -1112,6 +1190,9 @@ static __global__ __launch_bounds__(512) void skinny_mw_kernel(MwArgs a, std::co
                 for (int h = 0; h < CW; h++)
                     code[gi][t][h] = __builtin_nontemporal_load(
                         a.codes + (((size_t)tl[t] * G + min(gw + gi, G - 1)) * CW + h) * 64 + lane);
+        if constexpr (LORA) {
+            if (a.lora_staged && blockIdx.y == 0 && gw == NG * wk) lscale = ll.lora_slot_scale[slot];
+        }
         // the activations landed (the weight loads issued after them may stay in flight)
         constexpr int WL = ((F & F_BF16) ? 0 : 2) + ((F & F_ZP) ? 2 : 0) + 2 * NG * CW;
         __builtin_amdgcn_s_waitcnt((WL & 15) | ((WL >> 4) << 14) | (7 << 4) | (15 << 8));
@@ -1155,17 +1236,20 @@ static __global__ __launch_bounds__(512) void skinny_mw_kernel(MwArgs a, std::co
         }
     }
     if constexpr (LORA) {
-        if (wk == 0 && blockIdx.y == 0) {
-#pragma unroll
-            for (int t = 0; t < 2; t++) {
-                if (tile0 + t >= T) break;
-                f32x4 d = {0.0f, 0.0f, 0.0f, 0.0f};
-#pragma unroll
-                for (int r = 0; r < NR; r++) d[r] = acc[t][r];
-                lora_delta16<EPI == EPI_SILU>(ll, tile0 + t, 0, d);
-#pragma unroll
-                for (int r = 0; r < NR; r++) acc[t][r] = d[r];
+        if (blockIdx.y == 0) {  // the adapter's delta, on split 0
+            __builtin_amdgcn_s_waitcnt(0);
+            __syncthreads();  // every wave's staged words have landed
+            f32x4 d[2] = {{0.0f, 0.0f, 0.0f, 0.0f}, {0.0f, 0.0f, 0.0f, 0.0f}};
+            if (a.lora_staged) {
+                lora_share16<EPI == EPI_SILU>(ll, lst, lscale, tile0, T, wk, WK, d);
+            } else if (wk == 0) {
+                lora_delta16<EPI == EPI_SILU>(ll, tile0, 0, d[0]);
+                if (tile0 + 1 < T) lora_delta16<EPI == EPI_SILU>(ll, tile0 + 1, 0, d[1]);
             }
+#pragma unroll
+            for (int t = 0; t < 2; t++)
+#pragma unroll
+                for (int r = 0; r < NR; r++) acc[t][r] += d[t][r];
         }
     }
 #pragma unroll
@@ -1196,9 +1280,12 @@ template <int F, int EPI>
 static hipError_t mw_launch(const Launch& l, int wk) {
     constexpr int NG = mw_ng<F>();
     const int tiles = l.rows / TILE, G = l.cols / QG, nc = (G + NG - 1) / NG, gps = (nc + l.split - 1) / l.split * NG;
+    const size_t own = (size_t)wk * l.m * mt_xpitch<NG>() * 2 + (size_t)wk * l.m * 32 * 4;
+    const int lb = l.lora_rank ? lora16_bytes(l.lora_split, l.m, l.lora_cols, l.lora_rank) : 0;
+    const int staged = lb > 0 && lb <= LORA16_MAX && own + lb <= 160 * 1024 && ((uintptr_t)l.lora_b & 3) == 0;
     const MwArgs a{(const u32x4*)l.codes, l.scales, l.zeros, (const __bf16*)l.x, l.ldx, l.y, tiles, G, l.m, gps,
-                   l.nib_mask, l.bf16_magic};
-    const size_t lds = (size_t)wk * l.m * mt_xpitch<NG>() * 2 + (size_t)wk * l.m * 32 * 4;
+                   staged, l.nib_mask, l.bf16_magic};
+    const size_t lds = own + (staged ? lb : 0);
     const dim3 grid((tiles + 1) / 2, l.split), block(64 * wk);
     auto go = [&](auto NRc) {
         constexpr int NR = decltype(NRc)::value;

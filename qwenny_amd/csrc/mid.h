@@ -213,6 +213,10 @@ static __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2)))
     W w0, w1;
     stage(s0, 0);
     load(s0, w0);
+    if constexpr (LORA) {
+        // the adapter's delta (on split 0), shared by the wave rows, while the first step is on its way
+        if (EPI == EPI_SILU || blockIdx.y == 0) lora_item32<EPI == EPI_SILU, TB, 1>(ll, tile0, 0, acc, nullptr, 0, wk, WK);
+    }
     for (int s = s0; s < s1; s += 2) {
         __builtin_amdgcn_s_waitcnt(0);
         __syncthreads();
@@ -233,9 +237,6 @@ static __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2)))
         compute(s + 1, 1, w1);
     }
 
-    if constexpr (LORA) {
-        if (wk == 0 && (EPI == EPI_SILU || blockIdx.y == 0)) lora_item32<EPI == EPI_SILU, TB, 1>(ll, tile0, 0, acc);
-    }
     // one accumulator register (bv: token block bv / 16, register bv % 16) of the finished sums
     const int tile = tile0 + (l32 >> 4), out = tile * TILE + l16;
     const bool tile_ok = tile < T;
