@@ -14,12 +14,9 @@ using namespace qh;
 
 namespace {
 
-// v += x[0][i] + x[1][i] + .. + x[splits - 1][i], in that order; the partials load B at a time ahead of their adds
-// (the sum of 34 partials of a decode product is then 3-5 memory round trips, not 34). Decode sizes, where few
-// workgroups each wait on their loads: B = 16 (the 10-12 partials of most decode products in one round trip; 32
-// measured slower); streaming sizes: B = 8.
-template <int B = 8>
+// v += x[0][i] + x[1][i] + .. + x[splits - 1][i], in that order; the partials load 8 at a time ahead of their adds
 __device__ __forceinline__ void add_splits(float4& v, const float4* __restrict__ x, int splits, long n4, long i) {
+    constexpr int B = 8;
     for (int s0 = 0; s0 < splits; s0 += B) {
         float4 p[B];
 #pragma unroll
@@ -33,14 +30,36 @@ __device__ __forceinline__ void add_splits(float4& v, const float4* __restrict__
 
 // y [n][ld] = sum over s of x [s][n][ld] (from 0; h = nullptr), or h [n][ld] += that sum (h + x[0] first, as the
 // residual step adds); one thread per 4 columns (ld % 4 == 0), grid-stride over n * ld / 4
-template <int B>
 __global__ __launch_bounds__(256) void sum_parts_kernel(const float4* __restrict__ x, int splits, long n4, float4* y,
                                                         float4* h) {
     for (long i = (long)blockIdx.x * blockDim.x + threadIdx.x; i < n4; i += (long)gridDim.x * blockDim.x) {
         float4 v = h ? h[i] : make_float4(0.0f, 0.0f, 0.0f, 0.0f);
-        add_splits<B>(v, x, splits, n4, i);
+        add_splits(v, x, splits, n4, i);
         (h ? h : y)[i] = v;
     }
+}
+
+// The same sums at decode sizes: a thread per column and B partials of it in flight. Their time is the memory round trips
+// of each thread, not the bytes, so a quarter of the columns per thread buys 24 partials at once (34: two round trips
+// instead of three) and four times the waves. Graph replays after a kernel that writes the partials, us, against a thread
+// per 4 columns with 16 in flight: 5120 wide, 1 token, 12 / 19 / 34 partials 1.10 / 2.42 / 2.88 -> 1.05 / 1.90 / 2.29, 20
+// tokens 3.68 / 5.50 / 5.35 -> 3.60 / 5.06 / 4.77; 2560 wide, 5 tokens, 19 / 76 2.55 / 6.17 -> 2.04 / 5.23 (40 in flight
+// at 34 partials 2.48).
+template <int B>
+__global__ __launch_bounds__(64) void sum_cols_kernel(const float* __restrict__ x, int splits, long n1, float* y, float* h) {
+    const long i = (long)blockIdx.x * 64 + threadIdx.x;
+    if (i >= n1) return;
+    float v = h ? h[i] : 0.0f;
+    for (int s0 = 0; s0 < splits; s0 += B) {
+        float p[B];
+#pragma unroll
+        for (int j = 0; j < B; j++)
+            if (s0 + j < splits) p[j] = x[(size_t)(s0 + j) * n1 + i];
+#pragma unroll
+        for (int j = 0; j < B; j++)
+            if (s0 + j < splits) v += p[j];
+    }
+    (h ? h : y)[i] = v;
 }
 
 // add_rmsnorm takes one launch up to this many floats of partials per row (a row is one workgroup's, about 100 GB/s)
@@ -499,16 +518,16 @@ extern "C" int qh_lora_silu(void* stream, const float* xa, int split, int m_cols
     return lora_launch(stream, a, nullptr, y, (__bf16*)mid_bf16);
 }
 
-// launch sum_parts_kernel over n4 float4: workgroups of 64 threads for decode-sized rows (one float4 per thread over
-// 4x as many CUs), 256 otherwise
+// launch the sums over n4 float4: a thread per column below 64 Ki of them (decode sizes), else one per 4 columns
 static int sum_launch(hipStream_t s, const float* x, int splits, long n4, float* y, float* h) {
-    const unsigned t = n4 < 64l * 1024 ? 64 : 256, blocks = (unsigned)std::min<long>((n4 + t - 1) / t, 4096);
-    if (t == 64)
-        hipLaunchKernelGGL(sum_parts_kernel<16>, dim3(blocks), dim3(t), 0, s, (const float4*)x, splits, n4,
-                           (float4*)y, (float4*)h);
-    else
-        hipLaunchKernelGGL(sum_parts_kernel<8>, dim3(blocks), dim3(t), 0, s, (const float4*)x, splits, n4,
-                           (float4*)y, (float4*)h);
+    if (n4 < 64l * 1024) {
+        const dim3 grid((unsigned)((4 * n4 + 63) / 64));
+        if (splits <= 16) hipLaunchKernelGGL(sum_cols_kernel<16>, grid, dim3(64), 0, s, x, splits, 4 * n4, y, h);
+        else hipLaunchKernelGGL(sum_cols_kernel<24>, grid, dim3(64), 0, s, x, splits, 4 * n4, y, h);
+    } else {
+        hipLaunchKernelGGL(sum_parts_kernel, dim3((unsigned)std::min<long>((n4 + 255) / 256, 4096)), dim3(256), 0, s,
+                           (const float4*)x, splits, n4, (float4*)y, (float4*)h);
+    }
     return hipGetLastError() == hipSuccess ? QH_OK : QH_EHIP;
 }
 

@@ -1,4 +1,4 @@
-"""add_rmsnorm on both of its paths (one launch with the row in registers, or the partials' sum first): rows of one to
+"""The partials' sums at decode sizes (one thread per column) and beyond, and add_rmsnorm on both of its paths (one launch with the row in registers, or the partials' sum first): rows of one to
 four float4 per thread and a remainder, partials of every batch size, decode and streaming token counts, at the bound
 between the paths. The residual is bit-exact against the oracle's order, the bf16 output within one bf16 rounding of the
 f64 norm."""
@@ -7,7 +7,7 @@ import numpy as np
 import pytest
 
 import oracle
-from qwenny_amd import add_rmsnorm
+from qwenny_amd import add_rmsnorm, sum_parts
 from tests.helpers import bf16_out_err
 
 pytestmark = pytest.mark.gpu
@@ -32,3 +32,16 @@ def test_add_rmsnorm_paths(splits, n, hidden):
     want_h, want_y = oracle.add_rmsnorm(h, x, splits, w, 1e-6)
     assert np.array_equal(hd.cpu().numpy(), want_h)
     assert bf16_out_err(y.float().cpu().numpy(), want_y) <= 1e-5
+
+
+@pytest.mark.parametrize("splits,n,ld", [(1, 1, 4), (16, 1, 36), (17, 3, 20), (24, 1, 4096), (49, 2, 2560), (5, 64, 4092),
+                                         (5, 64, 4096), (17, 65, 4096)])
+def test_sum_parts_sizes(splits, n, ld):
+    import torch
+
+    print(f"sum_parts {splits}x{n}x{ld}", flush=True)
+    x = np.random.default_rng(splits + n).standard_normal((splits, n, ld)).astype(np.float32)
+    y = torch.full((n, ld), float("nan"), device="cuda")
+    sum_parts(None, torch.from_numpy(x).cuda(), splits, n, ld, y)
+    torch.cuda.synchronize()
+    assert np.array_equal(y.cpu().numpy(), oracle.sum_parts(x, splits))
