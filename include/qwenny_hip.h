@@ -174,9 +174,10 @@ int qh_mat_describe(const qh_mat* m, qh_mat_desc* out);
 /* Copy a device matrix's packed buffers back to the host (sizes from qh_mat_describe); zeros may be NULL. */
 int qh_mat_download(const qh_mat* m, void* codes, void* scales, void* zeros);
 
-/* Split-K factor a plain product of n tokens uses on m (core.rs Mat::split): the skinny kernel's K chunks where it
- * takes the product (qh_mat_kernel), 1-16 K slices (slices x tokens <= 2048) on the prefill kernel up to 512
- * tokens, 1 above. No launch; the same value qh_gemm returns. */
+/* Split-K factor a plain product of n tokens uses on m (core.rs Mat::split): the decode kernels' splits of K where they
+ * take the product (qh_mat_kernel: by token count, storage and size, from 2 to one per group of K), 1-16 K slices
+ * (slices x tokens <= 2048) on the prefill kernel up to 512 tokens, 1 above and for dense bf16 matrices of up to 256
+ * rows from 49 tokens. No launch; the same value qh_gemm returns. */
 int qh_mat_split(const qh_ctx* ctx, const qh_mat* m, size_t n);
 
 /* Which kernel a product of n tokens (qh_gemm's n, or n_out for QH_EPI_ARGMAX) with epilogue `epi` runs on m:
