@@ -14,7 +14,11 @@
 // after it: acc += s (D - (128 + z) sum_k x), where sum_k x comes from one more MFMA against ones per k32 step (shared
 // by the wave's tiles). K is split over the waves of a workgroup (reduced through LDS) and, for plain products, over
 // the grid (the split-K partials of the output contract). The activations are staged in LDS once per workgroup, or,
-// for one token of int4 without zero points, by each wave for itself (no workgroup barrier).
+// for one token of int4 without zero points, by each wave for itself (no workgroup barrier). Most decode products run
+// on kernels of their own: skinny_m1_kernel and skinny_mt_kernel (int4 split-K products of 1 and 2-8 tokens),
+// skinny_m1w_kernel (one-token int4 whole sums), skinny_mw_kernel (whole sums and small matrices of up to 16 tokens, every
+// storage) and mid_kernel (9-48 tokens, mid.h); skinny_kernel keeps the argmax of 2 and more tokens, int8 and bf16
+// split-K products of more than 384 tiles at 1-8 tokens, and the cases of 9-48 tokens in which it is ahead.
 //
 // prefill_kernel (m > 48, and those 33-48-token products): MFMA-bound. A workgroup computes up to 256 tokens x 256 outputs (8 waves of 256 x 32, or
 // 256 x 192 on 12 waves of 128 x 32, or smaller tiles for short steps); the activation tile goes global -> LDS directly
@@ -1099,7 +1103,10 @@ static __global__ __launch_bounds__(512) void skinny_mt_kernel(MtArgs a) {
 // wave taking every WK-th chunk of NG groups, 8 KiB of codes in flight) with skinny_mt_kernel's token rows (each wave
 // stages its tokens' rows of its chunk, 16 bytes apart; token 4 r + lane / 16 in row r of a lane's accumulators). The
 // waves' sums meet in LDS and are added in wave order. Plain products of small matrices run on it too, K cut into a few
-// splits over the grid (api.hip mw_partition). A last chunk of fewer than NG groups reads its last group again.
+// splits over the grid (api.hip mw_partition). A last chunk of fewer than NG groups reads its last group again (TAIL, for
+// group counts that are no multiple of NG: a form of its own, as leaving the unrolled groups early keeps the compiler
+// from overlapping them: without it the 27B step at 5 tokens with every plain product as whole rows 0.3146 -> 0.3046 ms,
+// a 27B layer at 5 tokens 59.7 -> 58.2 us, a 4B layer with zero points at 4 tokens 33.7 -> 33.2).
 // HBM-bound, and latency-bound in skinny_kernel, whose workgroups of 2-8 wave columns are few on matrices of this size
 // and walk K one staged super-chunk after another.
 struct MwArgs {
@@ -1120,7 +1127,7 @@ struct NoLora {};
 template <int F>
 __host__ __device__ constexpr int mw_ng() { return 4 / CodeWords<F>::N; }
 
-template <int F, int EPI, int NR, bool LORA>
+template <int F, int EPI, int NR, bool LORA, bool TAIL>
 static __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(
     LORA && ((F == F_I4 && NR == 1) || (F & F_I8)) ? 6 : 2))) void skinny_mw_kernel(
     MwArgs a, std::conditional_t<LORA, Launch, NoLora> ll) {
@@ -1156,7 +1163,7 @@ static __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(
     const __bf16* xrow0 = xw + min(((l16 & 3) << 2) | (l16 >> 2), M - 1) * XP + 8 * kq;
     const int g1 = min((int)(blockIdx.y + 1) * a.gps, G);
     for (int gw = blockIdx.y * a.gps + NG * wk; gw < g1; gw += NG * WK) {
-        const int col = min(gw * QG + 8 * lane, G * QG - 8);
+        const int col = TAIL ? min(gw * QG + 8 * lane, G * QG - 8) : gw * QG + 8 * lane;
         for (int r = 0; r < M; r++)
             if (NG == 4 || lane < 16 * NG)
                 __builtin_amdgcn_global_load_lds((const void*)(a.x + (size_t)r * a.ldx + col),
@@ -1189,7 +1196,7 @@ static __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(
 #pragma unroll
                 for (int h = 0; h < CW; h++)
                     code[gi][t][h] = __builtin_nontemporal_load(
-                        a.codes + (((size_t)tl[t] * G + min(gw + gi, G - 1)) * CW + h) * 64 + lane);
+                        a.codes + (((size_t)tl[t] * G + (TAIL ? min(gw + gi, G - 1) : gw + gi)) * CW + h) * 64 + lane);
         if constexpr (LORA) {
             if (a.lora_staged && blockIdx.y == 0 && gw == NG * wk) lscale = ll.lora_slot_scale[slot];
         }
@@ -1198,7 +1205,7 @@ static __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(
         __builtin_amdgcn_s_waitcnt((WL & 15) | ((WL >> 4) << 14) | (7 << 4) | (15 << 8));
 #pragma unroll
         for (int gi = 0; gi < NG; gi++) {
-            if (NG > 1 && gw + gi >= G) break;  // wave-uniform
+            if (TAIL && gw + gi >= G) break;  // wave-uniform
             u32x4 xa[4];
 #pragma unroll
             for (int j = 0; j < 4; j++) xa[j] = *(const u32x4*)(xrow0 + gi * QG + 32 * j);
@@ -1289,8 +1296,17 @@ static hipError_t mw_launch(const Launch& l, int wk) {
     const dim3 grid((tiles + 1) / 2, l.split), block(64 * wk);
     auto go = [&](auto NRc) {
         constexpr int NR = decltype(NRc)::value;
-        if (l.lora_rank) hipLaunchKernelGGL((skinny_mw_kernel<F, EPI, NR, true>), grid, block, lds, l.stream, a, l);
-        else hipLaunchKernelGGL((skinny_mw_kernel<F, EPI, NR, false>), grid, block, lds, l.stream, a, NoLora{});
+        auto form = [&](auto TAILc) {
+            constexpr bool TAIL = decltype(TAILc)::value;
+            if (l.lora_rank)
+                hipLaunchKernelGGL((skinny_mw_kernel<F, EPI, NR, true, TAIL>), grid, block, lds, l.stream, a, l);
+            else
+                hipLaunchKernelGGL((skinny_mw_kernel<F, EPI, NR, false, TAIL>), grid, block, lds, l.stream, a, NoLora{});
+        };
+        if constexpr (NG > 1) {
+            if (G % NG) return form(std::true_type{});
+        }
+        form(std::false_type{});
     };
     // accumulator rows per lane: ceil(m / 4)
     if (l.m <= 4) go(std::integral_constant<int, 1>{});

@@ -66,6 +66,28 @@ def test_silu(gemm, kind, n, k):
         assert bf16_out_err(out.float().cpu().numpy(), g / (1 + np.exp(-g)) * u) <= 1e-4, m
 
 
+@pytest.mark.parametrize("kind", ["i4", "i4z", "i4s32", "i8g"])
+@pytest.mark.parametrize("n,k", [(528, 512), (528, 640), (528, 1024), (48, 5120), (48, 4992)])
+def test_whole_chunks(gemm, kind, n, k):
+    """Whole sums of 2-16 tokens with the groups of K whole chunks of a wave and with a shorter last one."""
+    import torch
+
+    plain, want_of = _matrix(gemm, kind, n, k)
+    gated, _ = _matrix(gemm, kind, n, k, silu=True)
+    for m in (2, 4, 5, 8, 9, 16):
+        print(f"whole chunks {kind} {n}x{k} m={m}", flush=True)
+        x = activations(m, "x", m, k)
+        want = want_of(x)
+        g, u = want[:, :n // 2], want[:, n // 2:]
+        y = torch.full((1, m, n), float("nan"), dtype=torch.float32, device="cuda")
+        assert gemm.run_split(None, m, plain, to_dev(x), y, Epi.Plain, True) == 1
+        out = torch.full((m, n // 2), float("nan"), dtype=torch.bfloat16, device="cuda")
+        gemm.run(None, m, gated, to_dev(x), out, Epi.Silu)
+        torch.cuda.synchronize()
+        assert rel_err(y[0].double().cpu().numpy(), want) <= 1e-4, m
+        assert bf16_out_err(out.float().cpu().numpy(), g / (1 + np.exp(-g)) * u) <= 1e-4, m
+
+
 @pytest.mark.parametrize("kind", ["i4", "i8g", "bf16"])
 @pytest.mark.parametrize("n,k", [(528, 384), (24592, 256), (65552, 128)])
 def test_argmax_gathered_rows(gemm, kind, n, k):
