@@ -518,9 +518,13 @@ extern "C" int qh_lora_silu(void* stream, const float* xa, int split, int m_cols
     return lora_launch(stream, a, nullptr, y, (__bf16*)mid_bf16);
 }
 
-// launch the sums over n4 float4: a thread per column below 64 Ki of them (decode sizes), else one per 4 columns
+// launch the sums over n4 float4: a thread per column below 64 Ki of them (decode sizes) where the partials are more than
+// 4 (at most 16 Ki float4: more than 2), else one per 4 columns. Graph replays after a kernel that writes the partials,
+// us, a thread per 4 columns against one per column: 51200 columns, 2 / 4 / 8 / 20 partials 1.86 / 2.14 / 2.44 / 3.83
+// against 1.88 / 1.98 / 2.41 / 3.35; 163840 columns, 1 / 4 / 8 / 20 / 34 2.07 / 2.82 / 4.09 / 7.42 / 8.64 against 2.49 /
+// 3.18 / 3.86 / 6.70 / 7.68.
 static int sum_launch(hipStream_t s, const float* x, int splits, long n4, float* y, float* h) {
-    if (n4 < 64l * 1024) {
+    if (n4 < 64l * 1024 && splits > (n4 <= 16l * 1024 ? 2 : 4)) {
         const dim3 grid((unsigned)((4 * n4 + 63) / 64));
         if (splits <= 16) hipLaunchKernelGGL(sum_cols_kernel<16>, grid, dim3(64), 0, s, x, splits, 4 * n4, y, h);
         else hipLaunchKernelGGL(sum_cols_kernel<24>, grid, dim3(64), 0, s, x, splits, 4 * n4, y, h);

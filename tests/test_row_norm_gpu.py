@@ -35,7 +35,8 @@ def test_add_rmsnorm_paths(splits, n, hidden):
 
 
 @pytest.mark.parametrize("splits,n,ld", [(1, 1, 4), (16, 1, 36), (17, 3, 20), (24, 1, 4096), (49, 2, 2560), (5, 64, 4092),
-                                         (5, 64, 4096), (17, 65, 4096)])
+                                         (5, 64, 4096), (17, 65, 4096), (2, 3, 2560), (3, 16, 4096), (3, 16, 4100),
+                                         (4, 16, 4096), (4, 16, 4100), (5, 16, 4100)])
 def test_sum_parts_sizes(splits, n, ld):
     import torch
 
