@@ -583,7 +583,6 @@ int qh::gemm_with_scratch(qh_ctx* ctx, void* stream, const qh_mat* w, const void
         l.lora_split = lora->split;
         l.lora_cols = lora->m_cols;
         l.lora_rank = lora->rank;
-        if (l.narrow) l.narrow = 0, l.whole = 1;  // the prefill kernel, with as many partials
         l.lora_b = lora->b_f16;
         l.lora_tab = lora->tab;
         l.lora_tok_slot = lora->tok_slot;

@@ -215,7 +215,7 @@ static __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2)))
     load(s0, w0);
     if constexpr (LORA) {
         // the adapter's delta (on split 0), shared by the wave rows, while the first step is on its way
-        if (EPI == EPI_SILU || blockIdx.y == 0) lora_item32<EPI == EPI_SILU, TB, 1>(ll, tile0, 0, acc, nullptr, 0, wk, WK);
+        if (EPI == EPI_SILU || blockIdx.y == 0) lora_item32<EPI == EPI_SILU, TB, 1>(ll, tile0, 32 * TB * blockIdx.z, acc, nullptr, 0, wk, WK);
     }
     for (int s = s0; s < s1; s += 2) {
         __builtin_amdgcn_s_waitcnt(0);
@@ -353,6 +353,8 @@ static __global__ __launch_bounds__(64) void sum_narrow_kernel(const float* x, i
 // are a handful there, each walking all of K. Bound by the activations, read once; so K is split over the grid until
 // the launch has a few hundred workgroups, and a second launch (sum_narrow) adds the partials, kept in the stream-K
 // scratch, into one row of sums per token: split 1 to the caller (whose fused adapter epilogue then stages it in LDS).
+// An adapter of the product itself is added to split 0's sums before them, as in mid_kernel's other products, so that
+// outputs without a delta keep the order of their sums.
 // Kernel trace at 333 tokens, 32 x 5120 / 16 x 17408: 29.7 us (24 items) -> 6.3 + 4.8 / 6.4 + 4.8 us (55 / 187
 // workgroups, then the sum).
 template <int F>
@@ -371,9 +373,14 @@ static hipError_t narrow_launch(const Launch& l) {
     a.spp = (a.steps + l.narrow - 1) / l.narrow;
     const size_t lds = std::max((size_t)mid_xbytes(32, a.gs_shift) * (a.spp > 1 ? 2 : 1), (size_t)8 * 4096);
     const dim3 grid((pairs + wt - 1) / wt, l.narrow, (l.m + 31) / 32), block(64 * wt, wk);
-    if (wt == 4) hipLaunchKernelGGL((mid_kernel<F, EPI_PLAIN, 1, 4, false>), grid, block, lds, l.stream, a, NoLora{});
-    else if (wt == 2) hipLaunchKernelGGL((mid_kernel<F, EPI_PLAIN, 1, 2, false>), grid, block, lds, l.stream, a, NoLora{});
-    else hipLaunchKernelGGL((mid_kernel<F, EPI_PLAIN, 1, 1, false>), grid, block, lds, l.stream, a, NoLora{});
+    auto go = [&](auto WTc) {
+        constexpr int WT = decltype(WTc)::value;
+        if (l.lora_rank) hipLaunchKernelGGL((mid_kernel<F, EPI_PLAIN, 1, WT, true>), grid, block, lds, l.stream, a, l);
+        else hipLaunchKernelGGL((mid_kernel<F, EPI_PLAIN, 1, WT, false>), grid, block, lds, l.stream, a, NoLora{});
+    };
+    if (wt == 4) go(std::integral_constant<int, 4>{});
+    else if (wt == 2) go(std::integral_constant<int, 2>{});
+    else go(std::integral_constant<int, 1>{});
     if (hipError_t e = hipGetLastError(); e != hipSuccess || l.narrow == 1) return e;
     const size_t n4 = (size_t)l.m * l.rows / 4;
     hipLaunchKernelGGL(sum_narrow_kernel, dim3((unsigned)((n4 + 63) / 64)), dim3(64), 0, l.stream, l.sk_part, l.narrow, n4,
