@@ -137,3 +137,50 @@ def test_adapter(gemm):
             gemm.run_lora(None, m, mat, to_dev(x), out, Epi.Silu, lora)
             want = oracle.lora_silu(want_of(x)[:, row_order(n, True)], xa, 2, b.view(np.uint16), rank, tab, slot, scale, m)
             assert bf16_out_err(out.float().cpu().numpy(), want) <= 1e-3
+
+
+@pytest.mark.parametrize("kind", ["i4", "i4z", "i4s32", "i8", "i8g", "bf16"])
+@pytest.mark.parametrize("n,k,rank,split", [(528, 1280, 8, 1), (528, 640, 16, 3), (1072, 384, 64, 2), (528, 4096, 64, 4),
+                                            (6160, 512, 16, 2)])
+def test_adapter_forms(gemm, kind, n, k, rank, split):
+    """Every storage's adapter forms at decode sizes: odd tile counts, whole and shorter last chunks of K, each rank, xa
+    staged in LDS or read from memory (64 columns twice of 4 partials). Outputs whose delta is exactly zero (tokens of
+    slot scale 0; plain products: rows of an unadapted module) are the product's without adapter bit for bit."""
+    import torch
+
+    plain, want_of = _matrix(gemm, kind, n, k)
+    gated, _ = _matrix(gemm, kind, n, k, silu=True)
+    end = n // 2 + 3  # plain: the second module's rows, from inside a tile, have no adapter
+    tabs = {False: [end] + [2**31 - 1] * 3 + [rank, -1, -1, -1], True: [2**31 - 1] * 4 + [0, rank, -1, -1]}
+    for m in (1, 2, 4, 5, 8, 12, 16, 33, 48):
+        rng = np.random.default_rng(m)
+        xa = rng.standard_normal((split, m, 2 * rank)).astype(np.float32)
+        b = (rng.standard_normal((n, rank)) * 0.1).astype(np.float16)
+        slot, scale = rng.integers(0, 3, m).astype(np.int32), np.array([0.0, 0.5, 2.0], np.float32)
+        off = torch.from_numpy(scale[slot] == 0).cuda()
+        dev = [torch.from_numpy(np.ascontiguousarray(v)).cuda() for v in (xa, b.view(np.int16), slot, scale)]
+        x = activations(m, "x", m, k)
+        xd, base = to_dev(x), want_of(x)
+        for mat, silu, whole in ((plain, False, False), (plain, False, True), (gated, True, False)):
+            print(f"adapter {kind} {n}x{k} rank={rank} m={m} silu={silu} whole={whole}", flush=True)
+            tab = tabs[silu]
+            lora = (dev[0], split, 2 * rank, dev[1], rank, torch.tensor(tab, dtype=torch.int32, device="cuda"), dev[2],
+                    dev[3])
+            if silu:
+                y, ref = (torch.full((m, n // 2), float("nan"), dtype=torch.bfloat16, device="cuda") for _ in range(2))
+                gemm.run(None, m, mat, xd, ref, Epi.Silu)
+                gemm.run_lora(None, m, mat, xd, y, Epi.Silu, lora)
+                torch.cuda.synchronize()
+                want = oracle.lora_silu(base[:, row_order(n, True)], xa, split, b.view(np.uint16), rank, tab, slot, scale, m)
+                assert bf16_out_err(y.float().cpu().numpy(), want) <= 1e-3, m
+                assert torch.equal(y.view(torch.int16)[off], ref.view(torch.int16)[off]), m
+                continue
+            s = 1 if whole else mat.split(m)
+            y, ref = (torch.full((s, m, n), float("nan"), device="cuda") for _ in range(2))
+            assert gemm.run_split(None, m, mat, xd, ref, Epi.Plain, whole) == s
+            assert gemm.run_lora(None, m, mat, xd, y, Epi.Plain, lora, whole) == s
+            torch.cuda.synchronize()
+            want = oracle.lora_add(base, xa, split, b.view(np.uint16), rank, tab, slot, scale, m)
+            assert rel_err(y.double().sum(0).cpu().numpy(), want) <= 1e-4, (m, whole)
+            y, ref = y.view(torch.int32), ref.view(torch.int32)
+            assert torch.equal(y[:, off], ref[:, off]) and torch.equal(y[:, :, end:], ref[:, :, end:]), (m, whole)
