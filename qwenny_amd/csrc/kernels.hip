@@ -273,14 +273,16 @@ __device__ void lora_delta16(const Launch& a, int tile, int tok0, f32x4& d) {
 // The same delta of a tile pair for kernels whose waves' accumulators are summed afterwards, from LDS: each wave takes a
 // share of the steps of every module of tiles tile0, tile0 + 1, two at a time, into d[tile]. The pair's B rows and the
 // tokens' xa partials are staged when the kernel starts (lora_stage16, 4 bytes per lane global -> LDS, ahead of the
-// weights), the module table read there too, so that no chain of loads follows the last chunk. Kernel trace, us, against
-// one wave reading them from memory at the end: 27B [gate; up], rank 16, one token 25.5 -> 23.2; 4B with zero points, rank
-// 64, 5 tokens, [gate; up] 18.7 -> 16.2, down 12.8 -> 11.1. (At one token and for int8 the kernel is held to six waves per
-// SIMD, as without adapter: 26.3 us at five.)
+// weights), the module table read there too, so that no chain of loads follows the last chunk. None of it may be waited
+// for ahead of the weights, and the table must not live in scratch memory, as it did: us, one box, before -> after, [gate;
+// up] SwiGLU 34816 x 5120 int4 rank 16 at 1 / 5 tokens 25.7 / 26.2 -> 23.8 / 24.5, rank 64 at 8 49.5 -> 32.3 (two workgroups
+// to a CU: the waves' sums take the staged rows' place), int8 37.8 / 38.1 -> 35.8 / 37.2; (17408, 5120) int8 plain rank 16
+// 25.7 / 26.9 -> 18.9 / 19.9; 19456 x 2560 int4 rank 16 at one 12.0 -> 9.9.
 struct Lora16 {
     const float* xa;     // [split][m][cols]
     const _Float16* b;   // the tile pair's rows: [32][rank]
-    int end[3], off[4];  // the modules' end rows and first columns of xa
+    // the modules' end rows and first columns of xa, in scalar registers
+    int end0, end1, end2, off0, off1, off2, off3;
 };
 __host__ __device__ inline int lora16_bytes(int split, int m, int cols, int rank) {
     return ((split * m * cols * 4 + 255) & ~255) + 32 * rank * 2;
@@ -299,8 +301,9 @@ __device__ __forceinline__ Lora16 lora_stage16(const Launch& a, int tile0, uint8
     // the last pair of an odd tile count: its second tile's rows are clamped away (never used)
     const int rows = min(32, a.rows - tile0 * TILE);
     copy((const uint32_t*)(a.lora_b + (size_t)tile0 * TILE * a.lora_rank), rows * a.lora_rank / 2, lds + bx);
-    const int* const tab = a.lora_tab;
-    return Lora16{(const float*)lds, (const _Float16*)(lds + bx), {tab[0], tab[1], tab[2]}, {tab[4], tab[5], tab[6], tab[7]}};
+    // (read as constant memory: scalar loads, no vector load for the staged words to be waited for with)
+    const auto* const tab = (const __attribute__((address_space(4))) int*)(uintptr_t)a.lora_tab;
+    return Lora16{(const float*)lds, (const _Float16*)(lds + bx), tab[0], tab[1], tab[2], tab[4], tab[5], tab[6], tab[7]};
 }
 
 template <bool SILU>
@@ -310,15 +313,18 @@ __device__ void lora_share16(const Launch& a, const Lora16& st, float s, int til
     const int Q = a.lora_rank / 4;
     const int lane = threadIdx.x & 63, l16 = lane & 15, q = lane >> 4;
     const int tok = min(((l16 & 3) << 2) | (l16 >> 2), a.m - 1);
+    // (values of their own: a choice between the struct's fields would be one of addresses, and keep it in scratch memory)
+    const int off0 = __builtin_amdgcn_readfirstlane(st.off0), off1 = __builtin_amdgcn_readfirstlane(st.off1);
+    const int off2 = __builtin_amdgcn_readfirstlane(st.off2), off3 = __builtin_amdgcn_readfirstlane(st.off3);
     int n = 0;  // pairs of steps passed
 #pragma unroll
     for (int t = 0; t < 2; t++) {
         const int tile = tile0 + t, o = tile * TILE + l16;
         if (tile >= tiles) break;  // wave-uniform
-        auto module = [&](int r) { return SILU ? (r >> 3) & 1 : (r >= st.end[0]) + (r >= st.end[1]) + (r >= st.end[2]); };
+        auto module = [&](int r) { return SILU ? (r >> 3) & 1 : (r >= st.end0) + (r >= st.end1) + (r >= st.end2); };
         const int mod = module(o), mlo = module(tile * TILE), mhi = module(tile * TILE + TILE - 1);
         for (int m = mlo; m <= mhi; m++) {
-            const int c0 = m < 2 ? (m ? st.off[1] : st.off[0]) : (m == 2 ? st.off[2] : st.off[3]);
+            const int c0 = m < 2 ? (m ? off1 : off0) : (m == 2 ? off2 : off3);
             if (c0 < 0) continue;  // wave-uniform
             for (int i0 = 0; i0 < Q; i0 += C, n++) {
                 if (n % nshare != share) continue;
@@ -1128,8 +1134,7 @@ template <int F>
 __host__ __device__ constexpr int mw_ng() { return 4 / CodeWords<F>::N; }
 
 template <int F, int EPI, int NR, bool LORA, bool TAIL>
-static __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(
-    LORA && ((F == F_I4 && NR == 1) || (F & F_I8)) ? 6 : 2))) void skinny_mw_kernel(
+static __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2))) void skinny_mw_kernel(
     MwArgs a, std::conditional_t<LORA, Launch, NoLora> ll) {
     extern __shared__ __attribute__((aligned(16))) uint8_t smem[];
     constexpr int NG = mw_ng<F>(), XP = mt_xpitch<NG>(), CW = CodeWords<F>::N;
@@ -1139,7 +1144,9 @@ static __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(
     const int T = a.tiles, G = a.G, M = a.m;
     const int tile0 = blockIdx.x * 2, t1 = min(tile0 + 1, T - 1);
     __bf16* xw = (__bf16*)smem + (size_t)wk * M * XP;                // the wave's M staged rows
-    float* red = (float*)(smem + (size_t)WK * M * XP * 2);          // [WK][M][32]: each wave's sums
+    // [WK][M][32]: each wave's sums (with an adapter over the staged rows, whose place its operands take)
+    uint8_t* const past = smem + (size_t)WK * M * XP * 2;
+    float* red = (float*)(LORA ? smem : past);
     uint32_t magic;
     asm volatile("v_mov_b32 %0, %1" : "=v"(magic) : "s"(a.magic));
     const uint32_t mask = a.mask;
@@ -1150,7 +1157,7 @@ static __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(
     if constexpr (LORA) {
         if (blockIdx.y == 0 && a.lora_staged) {
             slot = ll.lora_tok_slot[min(((l16 & 3) << 2) | (l16 >> 2), M - 1)];
-            lst = lora_stage16(ll, tile0, (uint8_t*)(red + (size_t)WK * M * 32), wk, WK);
+            lst = lora_stage16(ll, tile0, past, wk, WK);
         }
     }
     const bf16x8 ones = __builtin_bit_cast(bf16x8, u32x4{0x3F803F80u, 0x3F803F80u, 0x3F803F80u, 0x3F803F80u});
@@ -1197,15 +1204,20 @@ static __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(
                 for (int h = 0; h < CW; h++)
                     code[gi][t][h] = __builtin_nontemporal_load(
                         a.codes + (((size_t)tl[t] * G + (TAIL ? min(gw + gi, G - 1) : gw + gi)) * CW + h) * 64 + lane);
-        if constexpr (LORA) {
-            if (a.lora_staged && blockIdx.y == 0 && gw == NG * wk) lscale = ll.lora_slot_scale[slot];
-        }
         // the activations landed (the weight loads issued after them may stay in flight). The LDS counter is waited for too
         // (nothing is pending on it): the compiler takes a global -> LDS load for one that may return out of order with
         // other vector loads until then, and would wait for every weight before the first MFMA (whole rows of int4 at 2
         // tokens, (5120, 4096) 6.3 -> 5.7 us, (5120, 17408) 12.7 -> 12.1; int8 at one 7.9 -> 7.2)
         constexpr int WL = ((F & F_BF16) ? 0 : 2) + ((F & F_ZP) ? 2 : 0) + 2 * NG * CW;
         __builtin_amdgcn_s_waitcnt((WL & 15) | ((WL >> 4) << 14) | (7 << 4));
+        if constexpr (LORA) {
+            // (the slot, loaded ahead of the activations, has landed too; taken here, not ahead of the loop, where its wait
+            // would come before the first weights)
+            if (a.lora_staged && blockIdx.y == 0 && gw == NG * wk) {
+                asm volatile("" : "+v"(slot));
+                lscale = ll.lora_slot_scale[slot];
+            }
+        }
 #pragma unroll
         for (int gi = 0; gi < NG; gi++) {
             if (TAIL && gw + gi >= G) break;  // wave-uniform
@@ -1246,9 +1258,9 @@ static __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(
         }
     }
     if constexpr (LORA) {
+        __builtin_amdgcn_s_waitcnt(0);
+        __syncthreads();  // every wave's staged words have landed, and its rows are read
         if (blockIdx.y == 0) {  // the adapter's delta, on split 0
-            __builtin_amdgcn_s_waitcnt(0);
-            __syncthreads();  // every wave's staged words have landed
             f32x4 d[2] = {{0.0f, 0.0f, 0.0f, 0.0f}, {0.0f, 0.0f, 0.0f, 0.0f}};
             if (a.lora_staged) {
                 lora_share16<EPI == EPI_SILU>(ll, lst, lscale, tile0, T, wk, WK, d);
@@ -1290,7 +1302,8 @@ template <int F, int EPI>
 static hipError_t mw_launch(const Launch& l, int wk) {
     constexpr int NG = mw_ng<F>();
     const int tiles = l.rows / TILE, G = l.cols / QG, nc = (G + NG - 1) / NG, gps = (nc + l.split - 1) / l.split * NG;
-    const size_t own = (size_t)wk * l.m * mt_xpitch<NG>() * 2 + (size_t)wk * l.m * 32 * 4;
+    static_assert(mt_xpitch<NG>() * 2 >= 32 * 4, "with an adapter the waves' sums take the staged rows' place");
+    const size_t own = (size_t)wk * l.m * mt_xpitch<NG>() * 2 + (l.lora_rank ? 0 : (size_t)wk * l.m * 32 * 4);
     const int lb = l.lora_rank ? lora16_bytes(l.lora_split, l.m, l.lora_cols, l.lora_rank) : 0;
     const int staged = lb > 0 && lb <= LORA16_MAX && own + lb <= 160 * 1024 && ((uintptr_t)l.lora_b & 3) == 0;
     const MwArgs a{(const u32x4*)l.codes, l.scales, l.zeros, (const __bf16*)l.x, l.ldx, l.y, tiles, G, l.m, gps,
