@@ -14,9 +14,9 @@ using namespace qh;
 
 namespace {
 
-// v += x[0][i] + x[1][i] + .. + x[splits - 1][i], in that order; the partials load 8 at a time ahead of their adds
+// v += x[0][i] + x[1][i] + .. + x[splits - 1][i], in that order; the partials load B at a time ahead of their adds
+template <int B = 8>
 __device__ __forceinline__ void add_splits(float4& v, const float4* __restrict__ x, int splits, long n4, long i) {
-    constexpr int B = 8;
     for (int s0 = 0; s0 < splits; s0 += B) {
         float4 p[B];
 #pragma unroll
@@ -30,21 +30,18 @@ __device__ __forceinline__ void add_splits(float4& v, const float4* __restrict__
 
 // y [n][ld] = sum over s of x [s][n][ld] (from 0; h = nullptr), or h [n][ld] += that sum (h + x[0] first, as the
 // residual step adds); one thread per 4 columns (ld % 4 == 0), grid-stride over n * ld / 4
+template <int B>
 __global__ __launch_bounds__(256) void sum_parts_kernel(const float4* __restrict__ x, int splits, long n4, float4* y,
                                                         float4* h) {
     for (long i = (long)blockIdx.x * blockDim.x + threadIdx.x; i < n4; i += (long)gridDim.x * blockDim.x) {
         float4 v = h ? h[i] : make_float4(0.0f, 0.0f, 0.0f, 0.0f);
-        add_splits(v, x, splits, n4, i);
+        add_splits<B>(v, x, splits, n4, i);
         (h ? h : y)[i] = v;
     }
 }
 
-// The same sums at decode sizes: a thread per column and B partials of it in flight. Their time is the memory round trips
-// of each thread, not the bytes, so a quarter of the columns per thread buys 24 partials at once (34: two round trips
-// instead of three) and four times the waves. Graph replays after a kernel that writes the partials, us, against a thread
-// per 4 columns with 16 in flight: 5120 wide, 1 token, 12 / 19 / 34 partials 1.10 / 2.42 / 2.88 -> 1.05 / 1.90 / 2.29, 20
-// tokens 3.68 / 5.50 / 5.35 -> 3.60 / 5.06 / 4.77; 2560 wide, 5 tokens, 19 / 76 2.55 / 6.17 -> 2.04 / 5.23 (40 in flight
-// at 34 partials 2.48).
+// The same sums a thread per column, B partials of it in flight: few columns, whose time is each thread's chain of memory
+// round trips and not the bytes (sum_launch chooses)
 template <int B>
 __global__ __launch_bounds__(64) void sum_cols_kernel(const float* __restrict__ x, int splits, long n1, float* y, float* h) {
     const long i = (long)blockIdx.x * 64 + threadIdx.x;
@@ -62,8 +59,10 @@ __global__ __launch_bounds__(64) void sum_cols_kernel(const float* __restrict__ 
     (h ? h : y)[i] = v;
 }
 
-// add_rmsnorm takes one launch up to this many floats of partials per row (a row is one workgroup's, about 100 GB/s)
-constexpr size_t AR_ROW_FLOATS = 40960;
+// up to 64 tokens add_rmsnorm takes one launch up to this many floats of partials per row (8 partials of 2560, 4 of 5120)
+constexpr size_t AR_ROW_FLOATS = 20480;
+// and spreads many partials over workgroups first below this many float4 (64 tokens of a 5120-wide row)
+constexpr size_t AR_SPREAD_BELOW = 64 * 1280;
 
 // y[t] = bf16(w * (h[t] / rms(h[t]))) with the row held in registers: each of the T threads loads its C float4 of h
 // and of w at once (one memory round trip), then the sum of squares and the output (H4 <= T * C)
@@ -518,18 +517,33 @@ extern "C" int qh_lora_silu(void* stream, const float* xa, int split, int m_cols
     return lora_launch(stream, a, nullptr, y, (__bf16*)mid_bf16);
 }
 
-// launch the sums over n4 float4: a thread per column below 64 Ki of them (decode sizes) where the partials are more than
-// 4 (at most 16 Ki float4: more than 2), else one per 4 columns. Graph replays after a kernel that writes the partials,
-// us, a thread per 4 columns against one per column: 51200 columns, 2 / 4 / 8 / 20 partials 1.86 / 2.14 / 2.44 / 3.83
-// against 1.88 / 1.98 / 2.41 / 3.35; 163840 columns, 1 / 4 / 8 / 20 / 34 2.07 / 2.82 / 4.09 / 7.42 / 8.64 against 2.49 /
-// 3.18 / 3.86 / 6.70 / 7.68.
-static int sum_launch(hipStream_t s, const float* x, int splits, long n4, float* y, float* h) {
-    if (n4 < 64l * 1024 && splits > (n4 <= 16l * 1024 ? 2 : 4)) {
-        const dim3 grid((unsigned)((4 * n4 + 63) / 64));
-        if (splits <= 16) hipLaunchKernelGGL(sum_cols_kernel<16>, grid, dim3(64), 0, s, x, splits, 4 * n4, y, h);
-        else hipLaunchKernelGGL(sum_cols_kernel<24>, grid, dim3(64), 0, s, x, splits, 4 * n4, y, h);
+// Launch the sums of n rows of ld floats (ld % 4 == 0). What bounds them at decode sizes is the memory round trips of a
+// thread (its partials over its loads in flight) and the waves that share them. Up to 4 partials: one round trip in any
+// form, and few large workgroups launch fastest, but for the smallest rows. More: a thread per column while the columns
+// are few (four times the waves); from 16 Ki, or where it meets the writer's caches, a thread per 4 columns in workgroups
+// of 64: workgroup b runs on XCD b mod 8, as did the decode products' workgroup b of 256 rows, so that with rows of a
+// multiple of 2048 each finds its 256 columns in the L2 that their product left them in. 16 or 24 partials are in flight;
+// from 512 Ki columns, where the CUs are full, workgroups of 256 with 8. Graph replays, us added to the product that writes
+// the partials (other forms): 8 partials, 8 Ki columns 2.2 (a thread per 4 columns 2.3), 4 rows of 4096 1.8 (per column
+// 2.1), 8 of 6144 1.9 (2.6), 48 of 8192 3.3 (7.6, workgroups of 256 7.5); 20, 8 of 6144 2.2 (3.6), 8 of 5120 2.9 (3.2, 4.6);
+// 34, 8 Ki 3.1 (4.2), 64 Ki 3.3 (4.1, 5.7), 128 Ki 5.0 (6.4, 7.6); 4, 64 Ki 2.4 (2.5), 512 Ki 4.2 (5.4, workgroups of 64 5.2).
+static int sum_launch(hipStream_t s, const float* x, int splits, size_t rows, size_t ld, float* y, float* h) {
+    const bool few = splits <= 16;
+    const long n = (long)(rows * ld), n4 = n / 4;
+    if (splits <= 4 ? n <= 16l * 1024 : n < 16l * 1024 && (rows <= 2 || ld % 2048)) {
+        const dim3 grid((unsigned)((n + 63) / 64));
+        if (few) hipLaunchKernelGGL(sum_cols_kernel<16>, grid, dim3(64), 0, s, x, splits, n, y, h);
+        else hipLaunchKernelGGL(sum_cols_kernel<24>, grid, dim3(64), 0, s, x, splits, n, y, h);
+    } else if (splits > 4 && n < 512l * 1024) {
+        const dim3 grid((unsigned)((n4 + 63) / 64));
+        if (few)
+            hipLaunchKernelGGL(sum_parts_kernel<16>, grid, dim3(64), 0, s, (const float4*)x, splits, n4, (float4*)y,
+                               (float4*)h);
+        else
+            hipLaunchKernelGGL(sum_parts_kernel<24>, grid, dim3(64), 0, s, (const float4*)x, splits, n4, (float4*)y,
+                               (float4*)h);
     } else {
-        hipLaunchKernelGGL(sum_parts_kernel, dim3((unsigned)std::min<long>((n4 + 255) / 256, 4096)), dim3(256), 0, s,
+        hipLaunchKernelGGL(sum_parts_kernel<8>, dim3((unsigned)std::min<long>((n4 + 255) / 256, 4096)), dim3(256), 0, s,
                            (const float4*)x, splits, n4, (float4*)y, (float4*)h);
     }
     return hipGetLastError() == hipSuccess ? QH_OK : QH_EHIP;
@@ -540,7 +554,7 @@ extern "C" int qh_sum_parts(void* stream, const float* x, int splits, size_t n, 
     if (!x || !y || splits < 1) return fail(QH_EINVAL, "sum_parts: null or %d splits", splits);
     if (ld % 4 || (uintptr_t)x % 16 || (uintptr_t)y % 16)
         return fail(QH_EINVAL, "sum_parts: rows of %zu floats must be a multiple of 4, buffers 16-byte aligned", ld);
-    if (sum_launch((hipStream_t)stream, x, splits, (long)(n * ld / 4), y, nullptr))
+    if (sum_launch((hipStream_t)stream, x, splits, n, ld, y, nullptr))
         return fail(QH_EHIP, "sum_parts launch failed");
     return QH_OK;
 }
@@ -552,20 +566,26 @@ extern "C" int qh_add_rmsnorm(void* stream, float* h, const float* x, int splits
     if (hidden == 0 || hidden % 4 || hidden > (1u << 24) || n > 0x7fffffffu || (uintptr_t)h % 16 ||
         (uintptr_t)x % 16 || (uintptr_t)w_next % 16)
         return fail(QH_EINVAL, "add_rmsnorm: hidden %zu must be a multiple of 4, f32 buffers 16-byte aligned", hidden);
-    // One launch with the row in registers (row_norm_kernel) unless a row has more partials than its workgroup loads at
-    // once (16, and AR_ROW_FLOATS in all) and the tokens are up to 64 (few workgroups): then the partials' sum over many
-    // workgroups first, the norm afterwards. Graph replays after a kernel that writes the partials, us, two launches
-    // against one: 5120 wide, 1 token, 1 / 4 / 8 / 12 partials 4.6 / 4.1 / 4.3 / 4.2 against 2.4 / 3.3 / 4.3 / 5.8, 20
-    // tokens 5.3 / 5.0 / 5.7 / 6.4 against 2.9 / 4.1 / 5.6 / 7.6; 2560 wide, 1 token, 4 / 12 / 16 / 19 3.8 / 3.8 / 3.9 /
-    // 4.2 against 2.3 / 3.4 / 3.7 / 4.5, 48 tokens 4.8 / 6.8 / 7.4 / 6.8 against 3.4 / 5.9 / 6.3 / 6.7; 5120 wide, 100
-    // tokens, 8 partials 9.2 against 7.4. Streaming sizes, against a workgroup of 256 threads that reads its row again to
-    // normalise it: 5120 wide, 333 tokens, 1 / 4 partials 8.7 / 10.5 -> 6.6 / 9.4, 2048 tokens 29.9 / 57.0 -> 24.7 / 54.5.
+    // One launch with the row in registers (row_norm_kernel), or the partials' sum over many workgroups first and the norm
+    // afterwards. Up to 64 tokens one launch reads a row's partials on as many CUs as there are tokens, and is ahead while
+    // they are few: us added to the product that writes them, one launch (two): 1024 wide 2 / 4 / 8 / 12 partials 2.9 / 3.2 /
+    // 3.2 / 3.8 (3.9 / 3.9 / 3.8 / 4.1) at one token; 2560 2 / 4 / 8 / 10 2.9 / 3.5 / 4.0 / 4.6 (4.2 / 4.2 / 4.2 / 4.3) at one,
+    // 4 / 8 / 10 3.5 / 4.7 / 5.2 (4.4 / 4.9 / 5.0) at 20; 4096 4 / 8 3.9 / 4.8 (4.4 / 4.3); 5120 2 / 4 / 8 3.8 / 4.5 / 5.6 (4.4
+    // / 4.5 / 4.4) at one, 4 / 8 / 16 5.3 / 7.7 / 8.4 (5.7 / 5.9 / 6.3) at 48.
+    // Above, the rows fill the chip and one launch reads everything once; more than 16 partials, or more than 8 of wide rows,
+    // run faster in small workgroups that take a row's columns in turn, or spread while the rows are few (600 tokens of
+    // 5120, 16 partials 37.8 us against 33.1; 256 of 1024, 34 partials 10.5 against 9.2).
     const size_t H4 = hidden / 4;
-    const bool stream_rows = n > 256;
-    if (H4 <= 1024 * 4 && (n > 64 || (splits <= 16 && (size_t)splits * hidden <= AR_ROW_FLOATS))) {
+    const bool one_row = splits <= 16 && (size_t)splits * hidden <= AR_ROW_FLOATS;
+    const bool many = splits > 16 || (splits > 8 && (H4 > 2048 || (H4 > 1024 && n > 256)));
+    if (H4 <= 1024 * 4 && (n <= 64 ? one_row : !many)) {
         // float4 per thread and partials loaded ahead: one column each where a workgroup holds them (the shortest chain),
-        // two, or four, and one partial at a time, at streaming sizes (more rows in flight per CU)
-        const int c = H4 > 2048 || n >= 1024 ? 4 : H4 > 1024 || stream_rows ? 2 : 1;
+        // two, or four; a partial at a time at streaming sizes (more rows in flight per CU)
+        const bool stream_rows = n > (H4 > 1024 ? 255 : 384);
+        const int c = H4 <= 256 || (H4 <= 1024 && splits > 8)        ? 1
+                      : H4 > 2048 || n >= (H4 > 1024 ? 512 : 1024) ? 4
+                      : H4 > 1024 || stream_rows                   ? 2
+                                                                   : 1;
         const unsigned t = (unsigned)(((H4 + c - 1) / c + 63) / 64 * 64);
         auto go = [&](auto Cc, auto Bc) {
             hipLaunchKernelGGL((row_norm_kernel<decltype(Cc)::value, decltype(Bc)::value>), dim3((unsigned)n), dim3(t), 0,
@@ -576,16 +596,18 @@ extern "C" int qh_add_rmsnorm(void* stream, float* h, const float* x, int splits
         using I4 = std::integral_constant<int, 4>;
         using I8 = std::integral_constant<int, 8>;
         using I16 = std::integral_constant<int, 16>;
-        if (c == 4) go(I4{}, I1{});
-        else if (c == 2) {
-            if (stream_rows || splits <= 2) go(I2{}, I1{});
+        if (c == 4) {
+            if (n > 64 || splits == 1) go(I4{}, I1{});
+            else go(I4{}, I2{});
+        } else if (c == 2) {
+            if (stream_rows || splits == 1) go(I2{}, I1{});
             else if (splits <= 4) go(I2{}, I4{});
             else go(I2{}, I8{});
         } else if (splits <= 4) go(I1{}, I4{});
-        else if (splits <= 8 || n > 64) go(I1{}, I8{});
+        else if (splits <= 8) go(I1{}, I8{});
         else go(I1{}, I16{});
-    } else if (splits > 1 && n <= 64) {
-        if (sum_launch((hipStream_t)stream, x, splits, (long)(n * H4), nullptr, h))
+    } else if (splits > 1 && (n <= 64 || n * H4 < AR_SPREAD_BELOW)) {
+        if (sum_launch((hipStream_t)stream, x, splits, n, hidden, nullptr, h))
             return fail(QH_EHIP, "add_rmsnorm launch failed");
         // the norm alone, a wide workgroup per token with the row in registers
         if (H4 <= 1024 * 4)
@@ -594,6 +616,9 @@ extern "C" int qh_add_rmsnorm(void* stream, float* h, const float* x, int splits
         else
             hipLaunchKernelGGL(add_rmsnorm_kernel<1024>, dim3((unsigned)n), dim3(1024), 0, (hipStream_t)stream, h, x,
                                0, (int)n, (int)hidden, w_next, (__bf16*)y_bf16, eps);
+    } else if (n <= 64) {  // (rows of more than 16384: few workgroups, wide ones)
+        hipLaunchKernelGGL(add_rmsnorm_kernel<1024>, dim3((unsigned)n), dim3(1024), 0, (hipStream_t)stream, h, x, splits,
+                           (int)n, (int)hidden, w_next, (__bf16*)y_bf16, eps);
     } else {
         hipLaunchKernelGGL(add_rmsnorm_kernel<256>, dim3((unsigned)n), dim3(256), 0, (hipStream_t)stream,
                            h, x, splits, (int)n, (int)hidden, w_next, (__bf16*)y_bf16, eps);

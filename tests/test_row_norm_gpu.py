@@ -46,3 +46,21 @@ def test_sum_parts_sizes(splits, n, ld):
     sum_parts(None, torch.from_numpy(x).cuda(), splits, n, ld, y)
     torch.cuda.synchronize()
     assert np.array_equal(y.cpu().numpy(), oracle.sum_parts(x, splits))
+
+
+@pytest.mark.parametrize("splits,n,hidden", [(8, 3, 2560), (9, 2, 2560), (4, 2, 5120), (5, 2, 5120), (16, 2, 1280),
+                                             (16, 2, 1284), (2, 3, 10240), (3, 3, 10240), (17, 70, 1024), (17, 70, 2560),
+                                             (9, 300, 5120), (9, 70, 8196), (16, 400, 1024), (8, 385, 2560), (3, 255, 5120),
+                                             (3, 256, 5120), (3, 1030, 128), (2, 1024, 2048), (2, 66, 16388), (1, 2, 16388),
+                                             (1, 512, 5120), (17, 17, 16388)])
+def test_add_rmsnorm_bounds(splits, n, hidden):
+    """The bounds between its paths: partials of a row in one launch, wide and narrow rows with many of them, streaming
+    token counts."""
+    test_add_rmsnorm_paths(splits, n, hidden)
+
+
+@pytest.mark.parametrize("splits,n,ld", [(4, 1, 16384), (4, 1, 16388), (5, 1, 40956), (5, 1, 40960), (16, 1, 40964),
+                                         (17, 1, 16380), (17, 1, 16384), (24, 2, 8196), (25, 3, 5464), (5, 128, 4092),
+                                         (5, 128, 4096), (17, 128, 4096)])
+def test_sum_parts_bounds(splits, n, ld):
+    test_sum_parts_sizes(splits, n, ld)
