@@ -35,6 +35,7 @@ struct qh_ctx {
     int pf_from;            // products from this many tokens take the prefill kernel (QH_PF_FROM, tuning; 49: off)
     int skinny_few;         // plain products with fewer 4-group waves than this many per CU take 1-group waves (0: by
                             // token count; QH_SKINNY_FEW, tuning)
+    bool tuned;             // one of the QH_SKINNY_* overrides is set: skinny_kernel, whose partition they are
 };
 
 int qh::ctx_device(const qh_ctx* ctx) { return ctx->device; }
@@ -47,6 +48,13 @@ static Scratch ctx_scratch(const qh_ctx* ctx) {
 static int env_int(const char* name, int dflt) {
     const char* v = getenv(name);
     return v && *v ? atoi(v) : dflt;
+}
+
+// Whether one of the decode partition's overrides is in the environment.
+static bool skinny_tuned() {
+    for (const char* n : {"QH_SKINNY_MAX_W", "QH_SKINNY_FILL", "QH_SKINNY_TILE_WAVES", "QH_SKINNY_PLAIN_WK", "QH_SKINNY_FEW"})
+        if (const char* v = getenv(n); v && *v) return true;
+    return false;
 }
 
 struct qh_mat {
@@ -107,7 +115,7 @@ extern "C" int qh_open(int device, qh_ctx** out) {
                       std::min(9, std::max(0, env_int("QH_PF_SHAPE", 0))), sk, std::max(0, env_int("QH_PF_SK", 1)),
                       std::min(4, std::max(1, env_int("QH_SKINNY_PLAIN_WK", 1))),
                       std::max(1, env_int("QH_PF_FROM", SKINNY_MAX_M + 1)),
-                      std::min(64, std::max(0, env_int("QH_SKINNY_FEW", 0)))};
+                      std::min(64, std::max(0, env_int("QH_SKINNY_FEW", 0))), skinny_tuned()};
     return QH_OK;
 }
 
@@ -275,13 +283,12 @@ extern "C" int qh_mat_download(const qh_mat* m, void* codes, void* scales, void*
     return QH_OK;
 }
 
-// The skinny kernel's K partition: waves per workgroup and grid split for a product of m tokens. Enough waves
-// (about 12 per CU) to keep HBM busy, at least a few groups per wave so that its pipeline fills; non-plain epilogues
-// need whole sums in one workgroup (split 1).
+// The decode kernels' K partition of a product of m tokens: waves per workgroup and grid split (non-plain epilogues need
+// whole sums in one workgroup: split 1), and which of them takes it (skinny_kernel and its lean forms where neither).
 struct Partition {
     int tile_waves, waves, split, groups_per_wave, tiles_per_wave;
-    bool mid = false;  // mid_kernel takes the product
-    bool mw = false;   // skinny_mw_kernel does (plain, split)
+    bool mid = false;  // mid_kernel
+    bool mw = false;   // skinny_mw_kernel
 };
 
 // mid_kernel's partition of a product of 9-48 tokens, false where skinny_kernel stays: wave columns of two tiles x wave
@@ -302,8 +309,6 @@ struct Partition {
 // - wave rows: as many as give about 16 waves per CU (tiles x rows / 2), which smaller matrices need more of.
 static bool mid_partition(const qh_ctx* ctx, const qh_mat* m, size_t tokens, bool plain, bool argmax, Partition* out) {
     if (tokens <= 8 || tokens > (size_t)SKINNY_MAX_M) return false;
-    // (tuning overrides of skinny_kernel's partition)
-    if (ctx->skinny_tile_waves || ctx->skinny_plain_wk != 1 || ctx->skinny_few) return false;
     const int T = (int)(m->rows / TILE), G = (int)(m->cols / QG), M = (int)tokens;
     const bool wide = is_i8(m->wt) || is_bf16(m->wt);  // formats of one group per wave and step
     int wt, wk, aim = 0;  // aim: workgroups a plain launch aims for
@@ -360,13 +365,35 @@ static bool mid_partition(const qh_ctx* ctx, const qh_mat* m, size_t tokens, boo
 // (17.4) / 22.0 (17.6) / 23.1 (18.5). One-token int4 and int4 of 320 tiles and more keep their lean kernels, whose
 // products alone are faster ((17408, 5120) at 5 tokens 17.7 (10.8) against 16.3 (11.9)).
 static bool mw_partition(const qh_ctx* ctx, const qh_mat* m, size_t tokens, Partition* out) {
-    if (tokens < 1 || tokens > 8 || ctx->skinny_tile_waves || ctx->skinny_plain_wk != 1 || ctx->skinny_few) return false;
+    if (tokens < 1 || tokens > 8) return false;
     const int T = (int)(m->rows / TILE), G = (int)(m->cols / QG);
     const bool wide = is_i8(m->wt) || is_bf16(m->wt);
     if (wide ? T > 384 : T >= 320 || tokens == 1) return false;
     const int ng = is_bf16(m->wt) ? 1 : is_i8(m->wt) ? 2 : 4;  // groups per wave (mw_ng)
     const int chunks = (G + ng - 1) / ng, want = std::min(chunks, G >= 48 ? 3 : 2), each = (chunks + want - 1) / want;
     *out = Partition{1, std::min(8, each), (chunks + each - 1) / each, ng, SKINNY_TILES, false, true};
+    return true;
+}
+
+// skinny_mw_kernel for whole sums (plain products asked for whole rows, SwiGLU): up to 8 tokens, and up to 16 where
+// mid_kernel's or skinny_kernel's larger workgroups are few: up to 512 tiles, and up to 12 tokens to 1536 tiles and for
+// int8. Same-box graph replays, us per product against skinny_kernel: SwiGLU at 1 / 2 / 5 / 8 tokens 34816 x 5120 int4 (18.0
+// on skinny_m1w_kernel) / 21.5 / 23.1 / 24.1 -> - / 18.7 / 19.7 / 21.5, int8 35.9 / 36.0 / 39.6 / 40.0 -> 31.0 / 30.8 / 32.3 /
+// 33.5, 19456 x 2560 int4 - / 12.2 / 14.4 / 14.6 -> - / 8.0 / 8.7 / 9.0, int8 16.6 / 17.3 / 20.9 / 21.2 -> 11.4 / 11.4 / 13.1 /
+// 13.5, bf16 20.1 / 21.0 / 28.7 / 28.8 -> 17.7 / 18.0 / 18.5 / 19.0; whole rows (5120, 6144) int8 12.5 / 13.4 / 33.3 / 33.9 ->
+// 8.4 / 8.7 / 9.2 / 9.6, bf16 16.0 / 16.8 / 48.6 / 48.9 -> 11.5 / 11.6 / 12.1 / 12.7. Beyond 8 tokens against mid_kernel, at 9
+// / 12 / 16: 4864 x 2432 int4 7.2 / 7.8 / 8.0 -> 5.6 / 6.1 / 5.9, 19456 x 2560 13.1 / 13.0 / 13.2 -> 9.6 / 11.9 / 15.0, 34816 x
+// 5120 27.6 / 28.7 / 29.0 -> 33.5 / 33.5 / 32.1 (its activations staged by every wave), int8 44.3 / 39.7 / 41.1 -> 34.7 / 36.8 /
+// 46.0. bf16 of one and two tokens, and int4 with fewer than 16 groups, stay on skinny_kernel where a workgroup per tile
+// pair gives some CUs two and most one, between 1 and 1.5 rounds of the chip: bf16 10240 rows, K 2560 / 5120 / 17408, 11.7 /
+// 21.6 / 66.8 against 12.4 / 23.3 / 75.8, int4 SwiGLU 9728 x 1024 at two 4.5 against 4.8.
+static bool mw_whole(const qh_ctx* ctx, const qh_mat* m, size_t tokens, Partition* out) {
+    const int T = (int)(m->rows / TILE), G = (int)(m->cols / QG), pairs = (T + 1) / 2;
+    if (tokens < 1 || tokens > (size_t)(T <= 512 ? 16 : T <= 1536 || is_i8(m->wt) ? 12 : 8)) return false;
+    if ((is_bf16(m->wt) || (!is_i8(m->wt) && G < 16)) && tokens <= 2 && pairs > ctx->cus && 2 * pairs <= 3 * ctx->cus) return false;
+    // a wave per chunk up to 8, beyond that the chunks dealt out in turn (kernels.hip mw_waves)
+    const int ng = is_bf16(m->wt) ? 1 : is_i8(m->wt) ? 2 : 4;
+    *out = Partition{1, std::min(8, (G + ng - 1) / ng), 1, ng, SKINNY_TILES, false, true};
     return true;
 }
 
@@ -379,10 +406,13 @@ static bool mw_partition(const qh_ctx* ctx, const qh_mat* m, size_t tokens, Part
 // partials the consumer sums). Other epilogues need whole sums in one workgroup: its wave rows split K (reduced
 // through LDS), as few as give the launch enough waves to fill the CUs, dividing the chunks evenly and fitting the wave
 // and LDS limits; longer K is walked in super-chunks.
-static Partition skinny_partition(const qh_ctx* ctx, const qh_mat* m, size_t tokens, bool plain,
-                                  bool argmax = false) {
-    if (Partition p; mid_partition(ctx, m, tokens, plain, argmax, &p)) return p;
-    if (Partition p; plain && mw_partition(ctx, m, tokens, &p)) return p;
+static Partition skinny_partition(const qh_ctx* ctx, const qh_mat* m, size_t tokens, int epi, int whole) {
+    const bool plain = epi == QH_EPI_PLAIN && !whole, argmax = epi == QH_EPI_ARGMAX;
+    if (!ctx->tuned) {
+        if (Partition p; !plain && !argmax && mw_whole(ctx, m, tokens, &p)) return p;
+        if (Partition p; mid_partition(ctx, m, tokens, plain, argmax, &p)) return p;
+        if (Partition p; plain && mw_partition(ctx, m, tokens, &p)) return p;
+    }
     const int tiles = (int)(m->rows / TILE), G = (int)(m->cols / QG);
     // tiles per wave: one for plain int8 and bf16 products of 1-2 tokens (8 KiB of one tile, half the registers of a
     // two-tile wave, 5 waves per SIMD for int8: same-box graph replays, int8 per channel 27B set at M = 1 5.39 -> 5.49
@@ -494,7 +524,7 @@ static Launch make_launch(const qh_ctx* ctx, const qh_mat* w, const void* x, siz
     l.whole = whole;
     l.skinny = use_skinny(ctx, w, m, epi, whole);
     if (l.skinny) {
-        Partition p = skinny_partition(ctx, w, m, epi == QH_EPI_PLAIN && !whole, epi == QH_EPI_ARGMAX);
+        Partition p = skinny_partition(ctx, w, m, epi, whole);
         l.mid = p.mid;
         l.mw = p.mw;
         l.tile_waves = p.tile_waves;
@@ -518,7 +548,7 @@ static Launch make_launch(const qh_ctx* ctx, const qh_mat* w, const void* x, siz
 extern "C" int qh_mat_split(const qh_ctx* ctx, const qh_mat* m, size_t n) {
     if (!ctx || !m) return fail(QH_EINVAL, "split: null");
     if (n == 0) return 1;
-    if (use_skinny(ctx, m, n, QH_EPI_PLAIN, 0)) return skinny_partition(ctx, m, n, true).split;
+    if (use_skinny(ctx, m, n, QH_EPI_PLAIN, 0)) return skinny_partition(ctx, m, n, QH_EPI_PLAIN, 0).split;
     if (n > (size_t)PF_KS_MAX_M || n > (1u << 24)) return 1;
     Launch l = make_launch(ctx, m, nullptr, m->cols, n, nullptr, nullptr, QH_EPI_PLAIN, nullptr, 0, nullptr,
                            ctx_scratch(ctx));
@@ -537,14 +567,14 @@ extern "C" size_t qh_part_len(const qh_ctx* ctx, const qh_mat* const* mats, size
     size_t len = 0;
     for (size_t i = 0; ctx && mats && i < count; i++) {
         if (!mats[i]) continue;
-        // decode sizes: the largest split x tokens over every token count the skinny kernel takes (its partition
-        // can depend on the token count, e.g. under QH_SKINNY_PLAIN_WK); prefill sizes up to PF_KS_MAX_M tokens: at
+        // decode sizes: the largest split x tokens over every token count the decode kernels take (their partition
+        // depends on the token count); prefill sizes up to PF_KS_MAX_M tokens: at
         // most PF_KS_MAX partials and PF_KS_ROWS partial rows; beyond: one
         size_t rows = std::max(max_tok, std::min((size_t)PF_KS_MAX * std::min(max_tok, (size_t)PF_KS_MAX_M),
                                                  (size_t)PF_KS_ROWS));
         for (size_t n = 1; n <= std::min(max_tok, (size_t)SKINNY_MAX_M); n++)
             if (use_skinny(ctx, mats[i], n, QH_EPI_PLAIN, 0))
-                rows = std::max(rows, (size_t)skinny_partition(ctx, mats[i], n, true).split * n);
+                rows = std::max(rows, (size_t)skinny_partition(ctx, mats[i], n, QH_EPI_PLAIN, 0).split * n);
         len = std::max(len, rows * mats[i]->rows);
     }
     return len;

@@ -1962,21 +1962,7 @@ static hipError_t skinny_epi(const Launch& l) {
         }
     }
     if constexpr (EPI != EPI_ARGMAX) {
-        // whole rows and SwiGLU products of up to 8 tokens, and of up to 16 where mid_kernel's or skinny_kernel's larger
-        // workgroups are few: up to 512 tiles, and up to 12 tokens to 1536 tiles and for int8. Same-box graph replays,
-        // us per product against skinny_kernel: SwiGLU at 1 / 2 / 5 / 8 tokens 34816 x 5120 int4 (18.0 on
-        // skinny_m1w_kernel) / 21.5 / 23.1 / 24.1 -> - / 18.7 / 19.7 / 21.5, int8 35.9 / 36.0 / 39.6 / 40.0 -> 31.0 /
-        // 30.8 / 32.3 / 33.5, 19456 x 2560 int4 - / 12.2 / 14.4 / 14.6 -> - / 8.0 / 8.7 / 9.0, int8 16.6 / 17.3 / 20.9 /
-        // 21.2 -> 11.4 / 11.4 / 13.1 / 13.5, bf16 20.1 / 21.0 / 28.7 / 28.8 -> 17.7 / 18.0 / 18.5 / 19.0; whole rows
-        // (5120, 6144) int8 12.5 / 13.4 / 33.3 / 33.9 -> 8.4 / 8.7 / 9.2 / 9.6, bf16 16.0 / 16.8 / 48.6 / 48.9 -> 11.5 /
-        // 11.6 / 12.1 / 12.7. Beyond 8 tokens against mid_kernel, at 9 / 12 / 16: 4864 x 2432 int4 7.2 / 7.8 / 8.0 ->
-        // 5.6 / 6.1 / 5.9, 19456 x 2560 13.1 / 13.0 / 13.2 -> 9.6 / 11.9 / 15.0, 34816 x 5120 27.6 / 28.7 / 29.0 ->
-        // 33.5 / 33.5 / 32.1 (its activations staged by every wave), int8 44.3 / 39.7 / 41.1 -> 34.7 / 36.8 / 46.0.
         if (l.mw) return mw_launch<F, EPI>(l, l.waves);
-        const int tiles = l.rows / TILE;
-        const int most = tiles <= 512 ? 16 : tiles <= 1536 || (F & F_I8) ? 12 : 8;
-        if (l.m <= most && (EPI == EPI_SILU || l.whole) && !l.xrows)
-            return mw_launch<F, EPI>(l, mw_waves((l.cols / QG + mw_ng<F>() - 1) / mw_ng<F>()));
     }
     if constexpr ((F == F_I4 || F == F_ZP) && EPI == EPI_PLAIN) {
         // the lean one-token kernel: the partition skinny_partition gives a plain one-token product (4 wave columns of

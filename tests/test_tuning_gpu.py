@@ -10,7 +10,7 @@ import pytest
 
 from qwenny_amd import Epi, Gemm, Mat
 from qwenny_amd.synth import activations
-from tests.helpers import make_quant, oracle_y, rel_err, to_dev
+from tests.helpers import bf16_out_err, make_quant, oracle_y, rel_err, to_dev
 
 pytestmark = pytest.mark.gpu
 
@@ -72,3 +72,38 @@ def test_part_len_covers_tuned_split(monkeypatch, pk):
         assert torch.isnan(y[n:]).all()
     finally:
         tuned.close()
+
+
+@pytest.mark.parametrize("epi,whole", [(Epi.Plain, True), (Epi.Silu, False)])
+@pytest.mark.parametrize("kind,m", [("i8", 1), ("i8", 5), ("i4", 5), ("i4", 12)])
+def test_overrides_reach_whole_sums(monkeypatch, kind, m, epi, whole):
+    """The overrides hold for products of whole sums too: one wave per workgroup (QH_SKINNY_MAX_W=1) sums K in one order,
+    16 waves and a fill no launch reaches in another, so that some last bits differ; both are within the bar."""
+    import torch
+
+    q = make_quant(970 + m, kind, 1024, 4096)
+    x = activations(971 + m, "x", m, 4096)
+    got = []
+    for env in ({"QH_SKINNY_MAX_W": "1"}, {"QH_SKINNY_MAX_W": "16", "QH_SKINNY_FILL": "64"}):
+        print(f"overrides {kind} m={m} {epi.name} {env}", flush=True)
+        for k_, v in env.items():
+            monkeypatch.setenv(k_, v)
+        tuned = Gemm.load(0)
+        try:
+            mat = Mat.stack(tuned, [q], silu=epi == Epi.Silu)
+            y = torch.full((m, 1024 if whole else 512), float("nan"), dtype=torch.float32 if whole else torch.bfloat16,
+                           device="cuda")
+            tuned.run_split(None, m, mat, to_dev(x), y, epi, whole)
+            torch.cuda.synchronize()
+            got.append(y.float().cpu().numpy())
+            del mat
+        finally:
+            tuned.close()
+    want = oracle_y(q, x)
+    if not whole:
+        g, u = want[:, :512], want[:, 512:]
+        want = g / (1 + np.exp(-g)) * u
+    for y in got:  # (SwiGLU: beyond one bf16 rounding of the output)
+        assert (rel_err if whole else bf16_out_err)(y, want) <= 1e-4
+    if whole:
+        assert not np.array_equal(got[0], got[1])
