@@ -354,23 +354,40 @@ static bool mid_partition(const qh_ctx* ctx, const qh_mat* m, size_t tokens, boo
     return true;
 }
 
-// skinny_mw_kernel's partition of a plain product of 1-8 tokens: two or three splits of K, few partials, the rest of K
-// over the workgroup's waves. A consumer's sum of the partials costs by their number (add_rmsnorm takes one launch up to
-// 16, fewer of wide rows), and small matrices leave skinny_kernel few waves per CU unless it writes a partial per group.
-// Taken by wide formats up to 384 tiles and by int4 up to 319 tiles from 2 tokens. Same-box graph replays, us with
-// add_rmsnorm (alone), skinny_kernel and its lean forms against this, at 1 / 4 / 8 tokens: (4096, 2560) int4 - / 10.6
-// (4.7) / 11.6 (5.3) -> - / 7.9 (4.9) / 8.2 (5.0), int8 9.7 (4.4) / 11.2 (5.3) / 11.5 (5.5) -> 8.5 (5.4) / 8.6 (5.5) / 8.9
-// (5.8); (9728, 2560) int4 - / 10.9 (5.2) / 11.4 (5.5) -> - / 9.6 (6.0) / 9.9 (6.2), bf16 17.4 (9.6) / 19.6 (10.9) / 20.1
-// (11.5) -> 13.3 (9.8) / 13.5 (9.9) / 13.8 (10.3); (17408, 5120) int8 23.1 (16.8) / 25.9 (19.1) / 26.3 (19.4) -> 21.7
-// (17.4) / 22.0 (17.6) / 23.1 (18.5). One-token int4 and int4 of 320 tiles and more keep their lean kernels, whose
-// products alone are faster ((17408, 5120) at 5 tokens 17.7 (10.8) against 16.3 (11.9)).
-static bool mw_partition(const qh_ctx* ctx, const qh_mat* m, size_t tokens, Partition* out) {
+// skinny_mw_kernel's partition of a plain product of 1-8 tokens, false where skinny_kernel (its lean forms; `split`
+// partials) stays: K over the workgroup's waves and a few splits. A consumer's sum of the partials costs by their number
+// (add_rmsnorm takes one launch up to 16, fewer of wide rows), and on small matrices skinny_kernel has waves enough only
+// with a partial per group.
+// The splits: the least that come within 10% of the fewest rounds of the chip (workgroups over CUs) times chunks of K in a
+// workgroup, two chunks or more each, so that the last round is not nearly empty: (17408, 1024) bf16 one token 3 splits 96
+// workgroups 11.9 us, 8 splits 8.2; (17408, 6144) int8 3 splits 2.25 rounds 24.2, 4 splits 3.0 21.1.
+// Taken where the product with its consumer is no slower than skinny_kernel's, either consumer (graph replays, us alone /
+// with add_rmsnorm / with sum_parts, skinny_kernel -> this):
+// - int4 of up to 319 tiles from 2 tokens, where skinny_kernel writes more than 16 partials: (2560, 4096) at 2 tokens 4.1 /
+//   9.1 / 6.7 -> 4.4 / 7.9 / 6.5, (17408, 1024) at 2 4.8 / 14.0 / 12.2 -> 5.3 / 8.8 / 7.4; with fewer it stays: (5120, 4096) at
+//   4, 10 partials, 5.3 / 9.5 / 7.2 against 5.5 / 9.1 / 7.6. One token and larger matrices keep the lean kernels: (5120,
+//   6144) at 4 5.9 / 10.2 / 7.7 against 6.5 / 11.2 / 8.6.
+// - wide formats up to 384 tiles: from 3 tokens, where skinny_kernel needs two rows of accumulators ((5120, 4096) int8 at 4
+//   7.9 / 12.0 / 9.8 -> 6.6 / 10.0 / 8.6, (17408, 1024) 7.9 / 13.2 / 11.1 -> 6.2 / 9.8 / 8.3), but for a short K on 320 tiles
+//   and more ((1024, 6144) at 8 4.6 / 9.1 / 6.5 against 4.9 / 9.8 / 7.2); at one and two from 32 groups ((17408, 5120) int8 at
+//   one 18.4 / 23.0 / 20.9 -> 18.4 / 22.6 / 20.5, (2560, 4096) 4.7 / 8.9 / 6.6 against 5.3 / 8.7 / 7.2).
+static bool mw_partition(const qh_ctx* ctx, const qh_mat* m, size_t tokens, int split, Partition* out) {
     if (tokens < 1 || tokens > 8) return false;
     const int T = (int)(m->rows / TILE), G = (int)(m->cols / QG);
     const bool wide = is_i8(m->wt) || is_bf16(m->wt);
-    if (wide ? T > 384 : T >= 320 || tokens == 1) return false;
+    if (!wide && (T >= 320 || tokens == 1 || split <= 16)) return false;
+    if (wide && (T > 384 || (tokens <= 2 ? G < 32 : T >= 320 && G < 16))) return false;
     const int ng = is_bf16(m->wt) ? 1 : is_i8(m->wt) ? 2 : 4;  // groups per wave (mw_ng)
-    const int chunks = (G + ng - 1) / ng, want = std::min(chunks, G >= 48 ? 3 : 2), each = (chunks + want - 1) / want;
+    const int chunks = (G + ng - 1) / ng, pairs = (T + 1) / 2;
+    auto cost = [&](int s) {
+        const int each = (chunks + s - 1) / s, wgs = pairs * ((chunks + each - 1) / each);
+        return each * ((wgs + ctx->cus - 1) / ctx->cus);
+    };
+    const int most = std::max(1, std::min(8, chunks / 2));
+    int lo = cost(most), want = std::min(2, most);
+    for (int s = want; s < most; s++) lo = std::min(lo, cost(s));
+    while (want < most && 10 * cost(want) > 11 * lo) want++;
+    const int each = (chunks + want - 1) / want;
     *out = Partition{1, std::min(8, each), (chunks + each - 1) / each, ng, SKINNY_TILES, false, true};
     return true;
 }
@@ -411,7 +428,6 @@ static Partition skinny_partition(const qh_ctx* ctx, const qh_mat* m, size_t tok
     if (!ctx->tuned) {
         if (Partition p; !plain && !argmax && mw_whole(ctx, m, tokens, &p)) return p;
         if (Partition p; mid_partition(ctx, m, tokens, plain, argmax, &p)) return p;
-        if (Partition p; plain && mw_partition(ctx, m, tokens, &p)) return p;
     }
     const int tiles = (int)(m->rows / TILE), G = (int)(m->cols / QG);
     // tiles per wave: one for plain int8 and bf16 products of 1-2 tokens (8 KiB of one tile, half the registers of a
@@ -435,6 +451,7 @@ static Partition skinny_partition(const qh_ctx* ctx, const qh_mat* m, size_t tok
         const int pk = ctx->skinny_plain_wk;
         if (pk > 1 && (G / ng) % pk == 0 && wt * pk <= (tokens > 16 ? 8 : 16))
             return Partition{wt, wt * pk, G / ng / pk, ng, tpw};
+        if (Partition p; !ctx->tuned && mw_partition(ctx, m, tokens, G / ng, &p)) return p;
         return Partition{wt, wt, G / ng, ng, tpw};
     }
     const size_t per_group = std::max<size_t>(tokens, 1) * QG * 2;  // LDS bytes of one group's activations
