@@ -302,23 +302,39 @@ struct Partition {
 //   activations, 8-20 partials: (17408, 5120) int4 at 9 / 16 / 24 21.9 / 24.8 / 30.4 -> 19.9 / 20.8 / 21.1. skinny_kernel
 //   stays for int4 of 320 tiles and more up to 16 tokens while its 4-group splits are few ((6144, 5120) at 9 / 16 11.7 /
 //   12.9 against 12.9 / 13.6), and from 33 tokens but on small matrices (18.6 against 19.7: two token blocks leave two
-//   waves per SIMD).
+//   waves per SIMD). It stays too where a step of eight wave rows is mostly past the end of a short K or its partials are
+//   few enough: fewer than 16 groups (int4 and, from 320 tiles or 33 tokens, wide formats; (1024, 8192) int4 at 32 tokens
+//   11.2 against 13.0 with add_rmsnorm, 8.2 against 10.0 with sum_parts); int4 up to 16 tokens of fewer than 32 groups, and
+//   below 320 tiles where it has waves enough with a partial per 4 groups ((9728, 2560) at 12 12.3 / 9.9 against 12.0 /
+//   10.5, (5120, 4096) 10.8 / 8.4 against 12.2 / 10.8), above 512 tiles ((17408, 17408) at 9 52.1 / 44.9 against 62.7 /
+//   55.9); int4 of 161-319 tiles with fewer than 48 groups and deep int4 on up to 128 tiles from 17 tokens ((17408, 1024) at
+//   32 14.9 / 12.5 against 14.9 / 13.5); int8 of 161-319 tiles with fewer than 32 groups ((2560, 4096) at 9 10.7 / 8.0 against
+//   10.6 / 9.0, not at 17-32 tokens), on up to 128 tiles from 33 (at 48 18.9 / 16.4 against 19.2 / 18.2), and from 320 tiles
+//   with fewer than 48 groups unless the workgroups fill their last round of the chip ((5120, 6144) at 20 16.1 / 13.5 against
+//   17.1 / 14.5 in 2.25 rounds, (5120, 8192) 22.4 / 19.5 against 17.9 / 15.6 in 2.0).
 // - whole sums: skinny_kernel where its 16-tile workgroups of 8-16 waves fill the chip, from 2000 tiles (int4 up to 16
-//   tokens 27.6 against 29.9; argmax above 32 tokens); below that its few workgroups leave the chip idle (4096 x 2560
-//   whole rows 16-34 against 8-16).
+//   tokens 27.6 against 29.9, above 24 tokens with fewer than 16 groups 12.5 against 13.6; bf16 up to 16 tokens 69.8
+//   against 77.2; argmax above 32 tokens); below that its few workgroups leave the chip idle (4096 x 2560 whole rows
+//   16-34 against 8-16).
 // - wave rows: as many as give about 16 waves per CU (tiles x rows / 2), which smaller matrices need more of.
 static bool mid_partition(const qh_ctx* ctx, const qh_mat* m, size_t tokens, bool plain, bool argmax, Partition* out) {
     if (tokens <= 8 || tokens > (size_t)SKINNY_MAX_M) return false;
+    const bool i8 = is_i8(m->wt);
     const int T = (int)(m->rows / TILE), G = (int)(m->cols / QG), M = (int)tokens;
     const bool wide = is_i8(m->wt) || is_bf16(m->wt);  // formats of one group per wave and step
     int wt, wk, aim = 0;  // aim: workgroups a plain launch aims for
     if (plain) {
         if (!wide) {
-            if (M > 32 ? T > 160 || G >= 64 : M <= 16 && T >= 320 && G < 96) return false;
+            if (M > 32 ? T > 160 || G >= 64 : M <= 16 && T >= 320 && (G < 96 || T > 512)) return false;
+            if (G < (M <= 16 ? 32 : 16) || (T > 160 && T < 320 && G < 48) || (M > 16 && T <= 128 && G >= 96)) return false;
+            if (M <= 16 && T < 320 && G % 4 == 0 && (T + 1) / 2 * (G / 4) >= 4 * ctx->cus) return false;
             if (M <= 16 && T < 320) wt = 1, wk = 8, aim = 240;
             else if (M <= 32 && T >= 320) wt = 8, wk = 1, aim = 240;
             else if (M <= 32 && T <= 128) wt = 1, wk = 4, aim = 256;
             else wt = 4, wk = 1, aim = G >= 64 ? 384 : 256;
+        } else if (M > 32 ? G < 16 || (i8 && (T <= 128 || (T > 160 && G < 32)))
+                          : T >= 320 ? G < 16 : i8 && M <= 16 && T > 160 && G < 32) {
+            return false;
         } else if (M > 32) {
             if (T <= 128) wt = 1, wk = 4, aim = 256;
             else if (T < 320) wt = 4, wk = 1, aim = G >= 64 ? 384 : 256;
@@ -330,11 +346,12 @@ static bool mid_partition(const qh_ctx* ctx, const qh_mat* m, size_t tokens, boo
         }
     } else if (wide) {
         if (M > 32 && argmax) return false;
+        if (!i8 && M <= 16 && T > 2000 && !argmax) return false;
         if (T <= 512) wt = 1, wk = M > 32 ? 4 : 8;
         else if (T <= 1536) wt = M > 32 ? 4 : M > 24 ? 2 : 1, wk = M > 24 ? 2 : 4;
         else wt = T <= 3000 || M > 32 ? 2 : 4, wk = 2;
     } else {
-        if (T > 2000 && (M <= 16 || M > 32)) return false;
+        if (T > 2000 && (M <= 16 || M > 32 || (M > 24 && G < 16 && !argmax))) return false;
         if (M > 32 && argmax) return false;
         if (T <= 512) wt = M > 24 ? 2 : 1, wk = M > 32 ? 2 : M > 16 ? 4 : 8;
         else if (T <= 1536) wt = 4, wk = 2;
@@ -349,6 +366,11 @@ static bool mid_partition(const qh_ctx* ctx, const qh_mat* m, size_t tokens, boo
         const int want = std::max(1, std::min(most, (aim + columns - 1) / columns));
         const int each = (steps + want - 1) / want;  // steps per split
         split = (steps + each - 1) / each;
+        // int8 from 320 tiles where skinny_kernel's partials are few: only in rounds of the chip that are nearly full
+        const int rounds = (columns * split + ctx->cus - 1) / ctx->cus;
+        if (i8 && aim == 480 && G < 48 && G % 4 == 0 && (T + 1) / 2 * (G / 4) >= 4 * ctx->cus &&
+            20 * columns * split < 19 * rounds * ctx->cus)
+            return false;
     }
     *out = Partition{wt, wt * wk, split, wide ? 1 : 2, SKINNY_TILES, true};
     return true;
