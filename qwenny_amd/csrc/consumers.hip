@@ -573,8 +573,8 @@ extern "C" int qh_add_rmsnorm(void* stream, float* h, const float* x, int splits
     // 4 / 8 / 10 3.5 / 4.7 / 5.2 (4.4 / 4.9 / 5.0) at 20; 4096 4 / 8 3.9 / 4.8 (4.4 / 4.3); 5120 2 / 4 / 8 3.8 / 4.5 / 5.6 (4.4
     // / 4.5 / 4.4) at one, 4 / 8 / 16 5.3 / 7.7 / 8.4 (5.7 / 5.9 / 6.3) at 48.
     // Above, the rows fill the chip and one launch reads everything once; more than 16 partials, or more than 8 of wide rows,
-    // run faster in small workgroups that take a row's columns in turn, or spread while the rows are few (600 tokens of
-    // 5120, 16 partials 37.8 us against 33.1; 256 of 1024, 34 partials 10.5 against 9.2).
+    // run faster in small workgroups that take a row's columns in turn, or spread while the rows are few and not narrow (600
+    // tokens of 5120, 16 partials 37.8 us against 33.1; 256 of 1024, 34 partials 10.5 and spread 15.7 against 9.2).
     const size_t H4 = hidden / 4;
     const bool one_row = splits <= 16 && (size_t)splits * hidden <= AR_ROW_FLOATS;
     const bool many = splits > 16 || (splits > 8 && (H4 > 2048 || (H4 > 1024 && n > 256)));
@@ -606,7 +606,7 @@ extern "C" int qh_add_rmsnorm(void* stream, float* h, const float* x, int splits
         } else if (splits <= 4) go(I1{}, I4{});
         else if (splits <= 8) go(I1{}, I8{});
         else go(I1{}, I16{});
-    } else if (splits > 1 && (n <= 64 || n * H4 < AR_SPREAD_BELOW)) {
+    } else if (splits > 1 && (n <= 64 || (H4 > 256 && n * H4 < AR_SPREAD_BELOW))) {
         if (sum_launch((hipStream_t)stream, x, splits, n, hidden, nullptr, h))
             return fail(QH_EHIP, "add_rmsnorm launch failed");
         // the norm alone, a wide workgroup per token with the row in registers
