@@ -319,17 +319,27 @@ template <int F, int EPI>
 static hipError_t mid_epi(const Launch& l) {
     auto go = [&](auto TBc) {
         constexpr int TB = decltype(TBc)::value;
-        if (l.tile_waves == 1) return mid_launch<F, EPI, TB, 1>(l);
+        // (the widths that mid_partition gives: 8 for split-K products, and int4 above 32 tokens 2 or 4 columns)
+        constexpr bool narrow = TB == 1 || mid_ng<F>() == 1;
         if (l.tile_waves == 4) return mid_launch<F, EPI, TB, 4>(l);
-        if constexpr (EPI == EPI_PLAIN) {  // 8 (split-K) or 2 (whole rows)
+        if (l.tile_waves == 2) return mid_launch<F, EPI, TB, 2>(l);
+        if constexpr (narrow) {
+            if (l.tile_waves == 1) return mid_launch<F, EPI, TB, 1>(l);
+        }
+        if constexpr (narrow && EPI == EPI_PLAIN) {
             if (l.tile_waves == 8) return mid_launch<F, EPI, TB, 8>(l);
         }
-        return l.tile_waves == 2 ? mid_launch<F, EPI, TB, 2>(l) : hipErrorInvalidConfiguration;
+        return hipErrorInvalidConfiguration;
     };
-    return l.m > 32 ? go(std::integral_constant<int, 2>{}) : go(std::integral_constant<int, 1>{});
+    if constexpr (EPI != EPI_ARGMAX) {  // (the argmax: up to 32 tokens)
+        if (l.m > 32) return go(std::integral_constant<int, 2>{});
+    }
+    return go(std::integral_constant<int, 1>{});
 }
 
-// y = the sum of `splits` partials of n4 float4 each, in order (y of any alignment)
+// y = the sum of `splits` partials of n4 float4 each, in order (y of any alignment). (A template, so that only the object
+// of the format that launches it holds it.)
+template <int F>
 static __global__ __launch_bounds__(64) void sum_narrow_kernel(const float* x, int splits, size_t n4, float* y) {
     const size_t i = (size_t)blockIdx.x * 64 + threadIdx.x;
     if (i >= n4) return;
@@ -383,7 +393,7 @@ static hipError_t narrow_launch(const Launch& l) {
     else go(std::integral_constant<int, 1>{});
     if (hipError_t e = hipGetLastError(); e != hipSuccess || l.narrow == 1) return e;
     const size_t n4 = (size_t)l.m * l.rows / 4;
-    hipLaunchKernelGGL(sum_narrow_kernel, dim3((unsigned)((n4 + 63) / 64)), dim3(64), 0, l.stream, l.sk_part, l.narrow, n4,
+    hipLaunchKernelGGL(sum_narrow_kernel<F>, dim3((unsigned)((n4 + 63) / 64)), dim3(64), 0, l.stream, l.sk_part, l.narrow, n4,
                        (float*)l.y);
     return hipGetLastError();
 }
