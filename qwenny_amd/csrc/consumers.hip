@@ -517,20 +517,21 @@ extern "C" int qh_lora_silu(void* stream, const float* xa, int split, int m_cols
     return lora_launch(stream, a, nullptr, y, (__bf16*)mid_bf16);
 }
 
-// Launch the sums of n rows of ld floats (ld % 4 == 0). What bounds them at decode sizes is the memory round trips of a
-// thread (its partials over its loads in flight) and the waves that share them. Up to 4 partials: one round trip in any
+// Launch the sums of `rows` rows of ld floats (ld % 4 == 0). What bounds them at decode sizes is the memory round trips of
+// a thread (its partials over its loads in flight) and the waves that share them. Up to 4 partials: one round trip in any
 // form, and few large workgroups launch fastest, but for the smallest rows. More: a thread per column while the columns
-// are few (four times the waves); from 16 Ki, or where it meets the writer's caches, a thread per 4 columns in workgroups
-// of 64: workgroup b runs on XCD b mod 8, as did the decode products' workgroup b of 256 rows, so that with rows of a
-// multiple of 2048 each finds its 256 columns in the L2 that their product left them in. 16 or 24 partials are in flight;
-// from 512 Ki columns, where the CUs are full, workgroups of 256 with 8. Graph replays, us added to the product that writes
-// the partials (other forms): 8 partials, 8 Ki columns 2.2 (a thread per 4 columns 2.3), 4 rows of 4096 1.8 (per column
-// 2.1), 8 of 6144 1.9 (2.6), 48 of 8192 3.3 (7.6, workgroups of 256 7.5); 20, 8 of 6144 2.2 (3.6), 8 of 5120 2.9 (3.2, 4.6);
-// 34, 8 Ki 3.1 (4.2), 64 Ki 3.3 (4.1, 5.7), 128 Ki 5.0 (6.4, 7.6); 4, 64 Ki 2.4 (2.5), 512 Ki 4.2 (5.4, workgroups of 64 5.2).
+// are few (four times the waves: 16 Ki, 64 Ki of one or two rows); else a thread per 4 columns in workgroups of 64, also
+// where that meets the writer's caches: workgroup b runs on XCD b mod 8, as did the decode products' workgroup b of 256
+// rows (3 tokens and more), so that with rows of a multiple of 2048 each finds its 256 columns in the L2 that their
+// product left them in. 16 or 24 partials are in flight; from 512 Ki columns, where the CUs are full, workgroups of 256
+// with 8. Graph replays, us added to the product that writes the partials (other forms): 8 partials, 8 Ki columns 2.2 (a
+// thread per 4 columns 2.3), 2 rows of 17408 2.3 (2.7), 4 rows of 4096 1.8 (per column 2.1), 8 of 6144 1.9 (2.6), 48 of
+// 8192 3.3 (7.6, workgroups of 256 7.5); 20, 8 of 6144 2.2 (3.6), 8 of 5120 2.9 (3.2, 4.6); 34, 8 Ki 3.1 (4.2), 64 Ki 3.3
+// (4.1, 5.7), 128 Ki 5.0 (6.4, 7.6); 4, 64 Ki 2.4 (2.5), 512 Ki 4.2 (5.4, workgroups of 64 5.2).
 static int sum_launch(hipStream_t s, const float* x, int splits, size_t rows, size_t ld, float* y, float* h) {
     const bool few = splits <= 16;
     const long n = (long)(rows * ld), n4 = n / 4;
-    if (splits <= 4 ? n <= 16l * 1024 : n < 16l * 1024 && (rows <= 2 || ld % 2048)) {
+    if (splits <= 4 ? n <= 16l * 1024 : rows <= 2 ? n < 64l * 1024 : n < 16l * 1024 && ld % 2048) {
         const dim3 grid((unsigned)((n + 63) / 64));
         if (few) hipLaunchKernelGGL(sum_cols_kernel<16>, grid, dim3(64), 0, s, x, splits, n, y, h);
         else hipLaunchKernelGGL(sum_cols_kernel<24>, grid, dim3(64), 0, s, x, splits, n, y, h);
