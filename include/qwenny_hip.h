@@ -175,7 +175,7 @@ int qh_mat_describe(const qh_mat* m, qh_mat_desc* out);
 int qh_mat_download(const qh_mat* m, void* codes, void* scales, void* zeros);
 
 /* Split-K factor a plain product of n tokens uses on m (core.rs Mat::split): the decode kernels' splits of K where they
- * take the product (qh_mat_kernel: by token count, storage and size, from 2 to one per group of K), 1-16 K slices
+ * take the product (by token count, storage and size, from 1 to one per group of K: cols / 128), 1-16 K slices
  * (slices x tokens <= 2048) on the prefill kernel up to 512 tokens, 1 above and for dense bf16 matrices of up to 256
  * rows from 49 tokens. No launch; the same value qh_gemm returns. */
 int qh_mat_split(const qh_ctx* ctx, const qh_mat* m, size_t n);
@@ -183,9 +183,11 @@ int qh_mat_split(const qh_ctx* ctx, const qh_mat* m, size_t n);
 /* Which kernel a product of n tokens (qh_gemm's n, or n_out for QH_EPI_ARGMAX) with epilogue `epi` runs on m:
  * QH_KERNEL_SKINNY (exact products of the dequantized weights) or QH_KERNEL_PREFILL (weights rounded to bf16 once;
  * both within the bf16-operand bound). No counterpart in the reference, whose Marlin kernel serves every token count:
- * for callers and tests that need to know which numerics a product has. The skinny kernel takes up to 48 tokens,
- * except split-K plain and SwiGLU products of int4 and grouped int8 matrices of at least 2^26 weights from 33
- * tokens. No launch. */
+ * for callers and tests that need to know which numerics a product has. QH_KERNEL_SKINNY, the decode kernels, takes up
+ * to 48 tokens, except split-K plain and SwiGLU products of int4 and grouped int8 matrices of at least 2^26 weights
+ * from 33 tokens. Plain products of dense bf16 matrices of up to 256 rows answer QH_KERNEL_PREFILL from 49 tokens like
+ * every other matrix, though they run on a decode kernel's blocks: the numerics are the same, such weights being
+ * products' operands as stored on either. No launch. */
 #define QH_KERNEL_SKINNY 1
 #define QH_KERNEL_PREFILL 2
 int qh_mat_kernel(const qh_ctx* ctx, const qh_mat* m, size_t n, int epi, int whole);

@@ -387,8 +387,10 @@ static bool mid_partition(const qh_ctx* ctx, const qh_mat* m, size_t tokens, boo
 // with add_rmsnorm / with sum_parts, skinny_kernel -> this):
 // - int4 of up to 319 tiles from 2 tokens, where skinny_kernel writes more than 16 partials: (2560, 4096) at 2 tokens 4.1 /
 //   9.1 / 6.7 -> 4.4 / 7.9 / 6.5, (17408, 1024) at 2 4.8 / 14.0 / 12.2 -> 5.3 / 8.8 / 7.4; with fewer it stays: (5120, 4096) at
-//   4, 10 partials, 5.3 / 9.5 / 7.2 against 5.5 / 9.1 / 7.6. One token and larger matrices keep the lean kernels: (5120,
-//   6144) at 4 5.9 / 10.2 / 7.7 against 6.5 / 11.2 / 8.6.
+//   4, 10 partials, 5.3 / 9.5 / 7.2 against 5.5 / 9.1 / 7.6. One token and larger matrices keep the lean kernels, the
+//   products alone being faster and most with a consumer too: (5120, 6144) at 4 5.9 / 10.2 / 7.7 against 6.5 / 11.2 / 8.6,
+//   (9728, 5120) at 2 7.0 / 12.0 / 9.5 against 7.7 / 12.0 / 9.8; the deepest would gain with one: (17408, 5120) at 8 12.1 /
+//   18.4 / 15.9 against 12.5 / 16.9 / 14.6.
 // - wide formats up to 384 tiles: from 3 tokens, where skinny_kernel needs two rows of accumulators ((5120, 4096) int8 at 4
 //   7.9 / 12.0 / 9.8 -> 6.6 / 10.0 / 8.6, (17408, 1024) 7.9 / 13.2 / 11.1 -> 6.2 / 9.8 / 8.3), but for a short K on 320 tiles
 //   and more ((1024, 6144) at 8 4.6 / 9.1 / 6.5 against 4.9 / 9.8 / 7.2); at one and two from 32 groups ((17408, 5120) int8 at

@@ -17,8 +17,9 @@
 // for one token of int4 without zero points, by each wave for itself (no workgroup barrier). Most decode products run
 // on kernels of their own: skinny_m1_kernel and skinny_mt_kernel (int4 split-K products of 1 and 2-8 tokens),
 // skinny_m1w_kernel (one-token int4 whole sums), skinny_mw_kernel (whole sums and small matrices of up to 16 tokens, every
-// storage) and mid_kernel (9-48 tokens, mid.h); skinny_kernel keeps the argmax of 2 and more tokens, int8 and bf16
-// split-K products of more than 384 tiles at 1-8 tokens, and the cases of 9-48 tokens in which it is ahead.
+// storage) and mid_kernel (9-48 tokens, mid.h); skinny_kernel keeps the argmax of 2 and more tokens, split-K products
+// whose partials are few or whose matrices are large, and the cases of 9-48 tokens in which it is ahead (api.hip
+// skinny_partition chooses, with both sides' times), and every decode product under the QH_SKINNY_* overrides.
 //
 // prefill_kernel (m > 48, and those 33-48-token products): MFMA-bound. A workgroup computes up to 256 tokens x 256 outputs (8 waves of 256 x 32, or
 // 256 x 192 on 12 waves of 128 x 32, or smaller tiles for short steps); the activation tile goes global -> LDS directly

@@ -107,3 +107,14 @@ def test_overrides_reach_whole_sums(monkeypatch, kind, m, epi, whole):
         assert (rel_err if whole else bf16_out_err)(y, want) <= 1e-4
     if whole:
         assert not np.array_equal(got[0], got[1])
+
+
+@pytest.mark.parametrize("kind", ["i4", "i8g"])
+@pytest.mark.parametrize("rows,cols", [(16, 128), (16, 17024), (2064, 1280), (4096, 2560), (5136, 1152)])
+def test_split_range(gemm, kind, rows, cols):
+    """qh_mat_split over the decode token counts: between 1 and a partial per group of K, and what part_len holds."""
+    print(f"split range {kind} {rows}x{cols}", flush=True)
+    mat = Mat.stack(gemm, [make_quant(980, kind, rows, cols)])
+    for m in range(1, 49):
+        assert 1 <= mat.split(m) <= cols // 128
+        assert mat.split(m) * m * rows <= gemm.part_len([mat], 48)
