@@ -1,4 +1,4 @@
-"""What the compiler gave the decode kernels, from the metadata of the code objects built here: the kernels of 1-48 tokens
+"""What the compiler gave the decode kernels, from the kernel descriptors of the code objects built here: the kernels of 1-48 tokens
 run without scratch memory. A register spill or a struct indexed at run time puts a chain of scratch accesses ahead of
 their first loads (an adapter's module table there made the int8 (17408, 5120) product of one token 1.4x slower)."""
 
@@ -6,14 +6,14 @@ import os
 import re
 import struct
 
-import msgpack
 import pytest
 
 from qwenny_amd.build import LIB
 
 
 def _kernels(path):
-    """{name: (scratch bytes, spilled VGPRs)} over the offload bundles of a shared library built by hipcc."""
+    """{name: scratch bytes} over the offload bundles of a shared library built by hipcc, from the kernel descriptors
+    (symbols NAME.kd: u32 LDS bytes, u32 scratch bytes per lane, ..)."""
     with open(path, "rb") as f:
         data = f.read()
     out = {}
@@ -28,16 +28,19 @@ def _kernels(path):
                 continue
             elf = data[at + offset:at + offset + size]
             assert elf[:4] == b"\x7fELF"
-            phoff, phentsize, phnum = struct.unpack_from("<Q", elf, 32)[0], *struct.unpack_from("<HH", elf, 54)
-            for i in range(phnum):
-                kind, _, off, _, _, filesz = struct.unpack_from("<IIQQQQ", elf, phoff + i * phentsize)
-                if kind != 4:  # PT_NOTE
+            shoff, shentsize, shnum = struct.unpack_from("<Q", elf, 40)[0], *struct.unpack_from("<HH", elf, 58)
+            # type, flags, address, offset, size, link of each section
+            sections = [struct.unpack_from("<IQQQQI", elf, shoff + i * shentsize + 4) for i in range(shnum)]
+            for kind, _, _, off, size, link in sections:
+                if kind != 11:  # SHT_DYNSYM
                     continue
-                namesz, descsz, _ = struct.unpack_from("<III", elf, off)
-                start = off + 12 + (namesz + 3) // 4 * 4
-                assert start + descsz <= off + filesz
-                for k in msgpack.unpackb(elf[start:start + descsz]).get("amdhsa.kernels", []):
-                    out[k[".name"]] = (k[".private_segment_fixed_size"], k[".vgpr_spill_count"])
+                names = sections[link][3]
+                for sym in range(off, off + size, 24):
+                    name, _, _, index, value, _ = struct.unpack_from("<IBBHQQ", elf, sym)
+                    name = elf[names + name:elf.index(b"\0", names + name)].decode()
+                    if name.endswith(".kd"):
+                        at_kd = value - sections[index][2] + sections[index][3]
+                        out[name[:-3]] = struct.unpack_from("<I", elf, at_kd + 4)[0]
     return out
 
 
@@ -47,4 +50,4 @@ def _kernels(path):
 def test_no_scratch(kernel):
     found = {n: r for n, r in _kernels(LIB).items() if f"{len(kernel)}{kernel}I" in n}
     assert found
-    assert not {n: r for n, r in found.items() if r != (0, 0)}
+    assert not {n: r for n, r in found.items() if r}
