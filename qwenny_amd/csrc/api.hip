@@ -291,6 +291,12 @@ struct Partition {
     bool mw = false;   // skinny_mw_kernel
 };
 
+// Dense bf16 matrices of few rows, an adapter's stacked A. Their consumer is the adapted product, each workgroup of which
+// reads all their partials, as a chain of loads where they do not fit its LDS: they keep few at every decode size (30 in
+// place of 2 at 2 tokens of 128 x 3840: a layer of hidden 3840 with a rank-64 adapter 55.8 -> 121 us; 6 in place of 2 at 8
+// tokens of 128 x 2176 49.0 -> 62.5).
+static bool adapter_rows(const qh_mat* m) { return is_bf16(m->wt) && m->rows / TILE <= (size_t)NARROW_TILES; }
+
 // mid_kernel's partition of a product of 9-48 tokens, false where skinny_kernel stays: wave columns of two tiles x wave
 // rows over K (each a group per step, two for int4) per workgroup, and the split of K over the grid (plain products
 // only, others need whole sums in one workgroup). Fitted to both kernels' times over 7 to 48 tokens, four formats and
@@ -332,8 +338,8 @@ static bool mid_partition(const qh_ctx* ctx, const qh_mat* m, size_t tokens, boo
             else if (M <= 32 && T >= 320) wt = 8, wk = 1, aim = 240;
             else if (M <= 32 && T <= 128) wt = 1, wk = 4, aim = 256;
             else wt = 4, wk = 1, aim = G >= 64 ? 384 : 256;
-        } else if (M > 32 ? G < 16 || (i8 && (T <= 128 || (T > 160 && G < 32)))
-                          : T >= 320 ? G < 16 : i8 && M <= 16 && T > 160 && G < 32) {
+        } else if (!adapter_rows(m) && (M > 32 ? G < 16 || (i8 && (T <= 128 || (T > 160 && G < 32)))
+                                               : T >= 320 ? G < 16 : i8 && M <= 16 && T > 160 && G < 32)) {
             return false;
         } else if (M > 32) {
             if (T <= 128) wt = 1, wk = 4, aim = 256;
@@ -398,16 +404,16 @@ static bool mid_partition(const qh_ctx* ctx, const qh_mat* m, size_t tokens, boo
 static bool mw_partition(const qh_ctx* ctx, const qh_mat* m, size_t tokens, int split, Partition* out) {
     if (tokens < 1 || tokens > 8) return false;
     const int T = (int)(m->rows / TILE), G = (int)(m->cols / QG);
-    const bool wide = is_i8(m->wt) || is_bf16(m->wt);
+    const bool wide = is_i8(m->wt) || is_bf16(m->wt), narrow = adapter_rows(m);
     if (!wide && (T >= 320 || tokens == 1 || split <= 16)) return false;
-    if (wide && (T > 384 || (tokens <= 2 ? G < 32 : T >= 320 && G < 16))) return false;
+    if (wide && !narrow && (T > 384 || (tokens <= 2 ? G < 32 : T >= 320 && G < 16))) return false;
     const int ng = is_bf16(m->wt) ? 1 : is_i8(m->wt) ? 2 : 4;  // groups per wave (mw_ng)
     const int chunks = (G + ng - 1) / ng, pairs = (T + 1) / 2;
     auto cost = [&](int s) {
         const int each = (chunks + s - 1) / s, wgs = pairs * ((chunks + each - 1) / each);
         return each * ((wgs + ctx->cus - 1) / ctx->cus);
     };
-    const int most = std::max(1, std::min(8, chunks / 2));
+    const int most = std::max(1, std::min(narrow ? (G >= 48 ? 3 : 2) : 8, chunks / 2));
     int lo = cost(most), want = std::min(2, most);
     for (int s = want; s < most; s++) lo = std::min(lo, cost(s));
     while (want < most && 10 * cost(want) > 11 * lo) want++;

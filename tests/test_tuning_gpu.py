@@ -9,7 +9,7 @@ import numpy as np
 import pytest
 
 from qwenny_amd import Epi, Gemm, Mat
-from qwenny_amd.synth import activations
+from qwenny_amd.synth import activations, f32_to_bf16
 from tests.helpers import bf16_out_err, make_quant, oracle_y, rel_err, to_dev
 
 pytestmark = pytest.mark.gpu
@@ -118,3 +118,14 @@ def test_split_range(gemm, kind, rows, cols):
     for m in range(1, 49):
         assert 1 <= mat.split(m) <= cols // 128
         assert mat.split(m) * m * rows <= gemm.part_len([mat], 48)
+
+
+@pytest.mark.parametrize("rows,cols", [(16, 1152), (32, 5120), (64, 17408), (128, 2176), (128, 3840), (256, 1024)])
+def test_adapter_partials(gemm, rows, cols):
+    """An adapter's stacked A (dense bf16, few rows) keeps few partials, which each workgroup of the adapted product reads:
+    up to 3 at 1-8 tokens, from 9 at most one per 4 groups of K (mid_kernel's wave rows)."""
+    print(f"adapter partials {rows}x{cols}", flush=True)
+    w = np.random.default_rng(rows).standard_normal((rows, cols)).astype(np.float32)
+    mat = Mat.new(gemm, f32_to_bf16(w), cols, int8=False)
+    for m in range(1, 49):
+        assert mat.split(m) <= (3 if m <= 8 else (cols // 128 + 3) // 4), m
