@@ -308,13 +308,14 @@ static bool adapter_rows(const qh_mat* m) { return is_bf16(m->wt) && m->rows / T
 //   activations, 8-20 partials: (17408, 5120) int4 at 9 / 16 / 24 21.9 / 24.8 / 30.4 -> 19.9 / 20.8 / 21.1. skinny_kernel
 //   stays for int4 of 320 tiles and more up to 16 tokens while its 4-group splits are few ((6144, 5120) at 9 / 16 11.7 /
 //   12.9 against 12.9 / 13.6), and from 33 tokens but on small matrices (18.6 against 19.7: two token blocks leave two
-//   waves per SIMD). It stays too where a step of eight wave rows is mostly past the end of a short K or its partials are
-//   few enough: fewer than 16 groups (int4 and, from 320 tiles or 33 tokens, wide formats; (1024, 8192) int4 at 32 tokens
-//   11.2 against 13.0 with add_rmsnorm, 8.2 against 10.0 with sum_parts); int4 up to 16 tokens of fewer than 32 groups, and
-//   below 320 tiles where it has waves enough with a partial per 4 groups ((9728, 2560) at 12 12.3 / 9.9 against 12.0 /
-//   10.5, (5120, 4096) 10.8 / 8.4 against 12.2 / 10.8), above 512 tiles ((17408, 17408) at 9 52.1 / 44.9 against 62.7 /
-//   55.9); int4 of 161-319 tiles with fewer than 48 groups and deep int4 on up to 128 tiles from 17 tokens ((17408, 1024) at
-//   32 14.9 / 12.5 against 14.9 / 13.5); int8 of 161-319 tiles with fewer than 32 groups ((2560, 4096) at 9 10.7 / 8.0 against
+//   waves per SIMD). It stays too where it has waves enough with a partial per 4 groups (`lean`): int4 up to 16 tokens below
+//   320 tiles ((9728, 2560) at 12 12.3 / 9.9 with add_rmsnorm / sum_parts against 12.0 / 10.5, (5120, 4096) 10.8 / 8.4
+//   against 12.2 / 10.8) and above 512 ((17408, 17408) at 9 52.1 / 44.9 against 62.7 / 55.9), from 17 tokens on 161-319
+//   tiles with fewer than 48 groups and deep on up to 128 tiles ((17408, 1024) at 32 14.9 / 12.5 against 14.9 / 13.5).
+//   Elsewhere on such matrices it would write a partial per group: layers at 12-28 tokens of hidden 2432 / 4352 / 1024 (19-43
+//   groups; 124 at 1024) 51.8 / 95.5 / 70.6 against 45.2 / 79.6 / 57.3 here, with one partial no consumer's sum at all.
+//   Few groups from 320 tiles stay with it: int4 from 17 tokens and wide formats of fewer than 16 ((1024, 8192) int4 at 32
+//   11.2 / 8.2 against 13.0 / 10.0); int8 of 161-319 tiles with fewer than 32 groups ((2560, 4096) at 9 10.7 / 8.0 against
 //   10.6 / 9.0, not at 17-32 tokens), on up to 128 tiles from 33 (at 48 18.9 / 16.4 against 19.2 / 18.2), and from 320 tiles
 //   with fewer than 48 groups unless the workgroups fill their last round of the chip ((5120, 6144) at 20 16.1 / 13.5 against
 //   17.1 / 14.5 in 2.25 rounds, (5120, 8192) 22.4 / 19.5 against 17.9 / 15.6 in 2.0).
@@ -331,9 +332,11 @@ static bool mid_partition(const qh_ctx* ctx, const qh_mat* m, size_t tokens, boo
     int wt, wk, aim = 0;  // aim: workgroups a plain launch aims for
     if (plain) {
         if (!wide) {
-            if (M > 32 ? T > 160 || G >= 64 : M <= 16 && T >= 320 && (G < 96 || T > 512)) return false;
-            if (G < (M <= 16 ? 32 : 16) || (T > 160 && T < 320 && G < 48) || (M > 16 && T <= 128 && G >= 96)) return false;
-            if (M <= 16 && T < 320 && G % 4 == 0 && (T + 1) / 2 * (G / 4) >= 4 * ctx->cus) return false;
+            // skinny_kernel has waves enough with a partial per 4 groups
+            const bool lean = G % 4 == 0 && (T + 1) / 2 * (G / 4) >= 4 * ctx->cus;
+            if (M > 32 ? T > 160 || G >= 64 : M <= 16 && T >= 320 && (G < 96 || (T > 512 && lean))) return false;
+            if (G < 16 && M > 16 && T >= 320) return false;
+            if (lean && (M <= 16 ? T < 320 : (T > 160 && T < 320 && G < 48) || (T <= 128 && G >= 96))) return false;
             if (M <= 16 && T < 320) wt = 1, wk = 8, aim = 240;
             else if (M <= 32 && T >= 320) wt = 8, wk = 1, aim = 240;
             else if (M <= 32 && T <= 128) wt = 1, wk = 4, aim = 256;
@@ -386,9 +389,10 @@ static bool mid_partition(const qh_ctx* ctx, const qh_mat* m, size_t tokens, boo
 // partials) stays: K over the workgroup's waves and a few splits. A consumer's sum of the partials costs by their number
 // (add_rmsnorm takes one launch up to 16, fewer of wide rows), and on small matrices skinny_kernel has waves enough only
 // with a partial per group.
-// The splits: the least that come within 10% of the fewest rounds of the chip (workgroups over CUs) times chunks of K in a
+// The splits: the least that come within 30% of the fewest rounds of the chip (workgroups over CUs) times chunks of K in a
 // workgroup, two chunks or more each, so that the last round is not nearly empty: (17408, 1024) bf16 one token 3 splits 96
-// workgroups 11.9 us, 8 splits 8.2; (17408, 6144) int8 3 splits 2.25 rounds 24.2, 4 splits 3.0 21.1.
+// workgroups 11.9 us, 8 splits 8.2; (17408, 6144) int8 3 splits 2.25 rounds 24.2, 4 splits 3.0 21.1. (Within
+// 10%, 5 in place of 2 for (5120, 3200) bf16 at 5 tokens, a layer 42.6 us became 44.5: the consumer reads them.)
 // Taken where the product with its consumer is no slower than skinny_kernel's, either consumer (graph replays, us alone /
 // with add_rmsnorm / with sum_parts, skinny_kernel -> this):
 // - int4 of up to 319 tiles from 2 tokens, where skinny_kernel writes more than 16 partials: (2560, 4096) at 2 tokens 4.1 /
@@ -400,13 +404,14 @@ static bool mid_partition(const qh_ctx* ctx, const qh_mat* m, size_t tokens, boo
 // - wide formats up to 384 tiles: from 3 tokens, where skinny_kernel needs two rows of accumulators ((5120, 4096) int8 at 4
 //   7.9 / 12.0 / 9.8 -> 6.6 / 10.0 / 8.6, (17408, 1024) 7.9 / 13.2 / 11.1 -> 6.2 / 9.8 / 8.3), but for a short K on 320 tiles
 //   and more ((1024, 6144) at 8 4.6 / 9.1 / 6.5 against 4.9 / 9.8 / 7.2); at one and two from 32 groups ((17408, 5120) int8 at
-//   one 18.4 / 23.0 / 20.9 -> 18.4 / 22.6 / 20.5, (2560, 4096) 4.7 / 8.9 / 6.6 against 5.3 / 8.7 / 7.2).
+//   one 18.4 / 23.0 / 20.9 -> 18.4 / 22.6 / 20.5) and where skinny_kernel writes more than 16 partials (layers of hidden 2176
+//   / 3840 int8 at two, 21-27 groups, 36.3 / 40.1 -> 34.6 / 37.7).
 static bool mw_partition(const qh_ctx* ctx, const qh_mat* m, size_t tokens, int split, Partition* out) {
     if (tokens < 1 || tokens > 8) return false;
     const int T = (int)(m->rows / TILE), G = (int)(m->cols / QG);
     const bool wide = is_i8(m->wt) || is_bf16(m->wt), narrow = adapter_rows(m);
     if (!wide && (T >= 320 || tokens == 1 || split <= 16)) return false;
-    if (wide && !narrow && (T > 384 || (tokens <= 2 ? G < 32 : T >= 320 && G < 16))) return false;
+    if (wide && !narrow && (T > 384 || (tokens <= 2 ? G < 32 && split <= 16 : T >= 320 && G < 16))) return false;
     const int ng = is_bf16(m->wt) ? 1 : is_i8(m->wt) ? 2 : 4;  // groups per wave (mw_ng)
     const int chunks = (G + ng - 1) / ng, pairs = (T + 1) / 2;
     auto cost = [&](int s) {
@@ -416,7 +421,7 @@ static bool mw_partition(const qh_ctx* ctx, const qh_mat* m, size_t tokens, int 
     const int most = std::max(1, std::min(narrow ? (G >= 48 ? 3 : 2) : 8, chunks / 2));
     int lo = cost(most), want = std::min(2, most);
     for (int s = want; s < most; s++) lo = std::min(lo, cost(s));
-    while (want < most && 10 * cost(want) > 11 * lo) want++;
+    while (want < most && 10 * cost(want) > 13 * lo) want++;
     const int each = (chunks + want - 1) / want;
     *out = Partition{1, std::min(8, each), (chunks + each - 1) / each, ng, SKINNY_TILES, false, true};
     return true;
