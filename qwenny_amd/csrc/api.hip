@@ -395,7 +395,8 @@ static bool mid_partition(const qh_ctx* ctx, const qh_mat* m, size_t tokens, boo
 // 10%, 5 in place of 2 for (5120, 3200) bf16 at 5 tokens, a layer 42.6 us became 44.5: the consumer reads them.)
 // Taken where the product with its consumer is no slower than skinny_kernel's, either consumer (graph replays, us alone /
 // with add_rmsnorm / with sum_parts, skinny_kernel -> this):
-// - int4 of up to 319 tiles from 2 tokens, where skinny_kernel writes more than 16 partials: (2560, 4096) at 2 tokens 4.1 /
+// - int4 of up to 319 tiles from 2 tokens, where skinny_kernel writes more than 16 partials, or one per group (a layer of
+//   hidden 2816 at two, 13 and 16 groups, 30.6 -> 28.4): (2560, 4096) at 2 tokens 4.1 /
 //   9.1 / 6.7 -> 4.4 / 7.9 / 6.5, (17408, 1024) at 2 4.8 / 14.0 / 12.2 -> 5.3 / 8.8 / 7.4; with fewer it stays: (5120, 4096) at
 //   4, 10 partials, 5.3 / 9.5 / 7.2 against 5.5 / 9.1 / 7.6. One token and larger matrices keep the lean kernels, the
 //   products alone being faster and most with a consumer too: (5120, 6144) at 4 5.9 / 10.2 / 7.7 against 6.5 / 11.2 / 8.6,
@@ -410,7 +411,7 @@ static bool mw_partition(const qh_ctx* ctx, const qh_mat* m, size_t tokens, int 
     if (tokens < 1 || tokens > 8) return false;
     const int T = (int)(m->rows / TILE), G = (int)(m->cols / QG);
     const bool wide = is_i8(m->wt) || is_bf16(m->wt), narrow = adapter_rows(m);
-    if (!wide && (T >= 320 || tokens == 1 || split <= 16)) return false;
+    if (!wide && (T >= 320 || tokens == 1 || (split <= 16 && split < G))) return false;
     if (wide && !narrow && (T > 384 || (tokens <= 2 ? G < 32 && split <= 16 : T >= 320 && G < 16))) return false;
     const int ng = is_bf16(m->wt) ? 1 : is_i8(m->wt) ? 2 : 4;  // groups per wave (mw_ng)
     const int chunks = (G + ng - 1) / ng, pairs = (T + 1) / 2;
