@@ -520,9 +520,10 @@ extern "C" int qh_lora_silu(void* stream, const float* xa, int split, int m_cols
 // Launch the sums of `rows` rows of ld floats (ld % 4 == 0). What bounds them at decode sizes is the memory round trips of
 // a thread (its partials over its loads in flight) and the waves that share them. Up to 4 partials: one round trip in any
 // form, and few large workgroups launch fastest, but for the smallest rows. More: a thread per column while the columns
-// are few (four times the waves: 16 Ki, 64 Ki of one or two rows, 256 Ki with more than 64 partials, three round trips: a
-// layer with 94 of 46 rows of 1280 56.6 us -> 55.7, 81 of 34 rows of 3200 83.1 -> 82.1); else a thread per 4 columns in workgroups of 64, also
-// where that meets the writer's caches: workgroup b runs on XCD b mod 8, as did the decode products' workgroup b of 256
+// are few (four times the waves: 16 Ki, 64 Ki of one or two rows), and for widths that are no multiple of 2048 also from 64
+// to 256 Ki, or with more than 64 partials (layers, us, a thread per 4 columns against this: 12 partials of 20 rows of 5120,
+// twice, 82.8 / 82.3, 27 and 81 of 44 rows of 3456 1.8% slower, 94 of 46 rows of 1280 56.6 / 55.7); else
+// a thread per 4 columns in workgroups of 64, also where that meets the writer's caches: workgroup b runs on XCD b mod 8, as did the decode products' workgroup b of 256
 // rows (3 tokens and more), so that with rows of a multiple of 2048 each finds its 256 columns in the L2 that their
 // product left them in. 16 or 24 partials are in flight; from 512 Ki columns, where the CUs are full, workgroups of 256
 // with 8. Graph replays, us added to the product that writes the partials (other forms): 8 partials, 8 Ki columns 2.2 (a
@@ -532,7 +533,8 @@ extern "C" int qh_lora_silu(void* stream, const float* xa, int split, int m_cols
 static int sum_launch(hipStream_t s, const float* x, int splits, size_t rows, size_t ld, float* y, float* h) {
     const bool few = splits <= 16;
     const long n = (long)(rows * ld), n4 = n / 4;
-    if (splits <= 4 ? n <= 16l * 1024 : rows <= 2 ? n < 64l * 1024 : n < (splits > 64 ? 256l : 16l) * 1024 && ld % 2048) {
+    const bool cols = n < 16l * 1024 || (n < 256l * 1024 && (splits > 64 || n >= 64l * 1024));
+    if (splits <= 4 ? n <= 16l * 1024 : rows <= 2 ? n < 64l * 1024 : cols && ld % 2048) {
         const dim3 grid((unsigned)((n + 63) / 64));
         if (few) hipLaunchKernelGGL(sum_cols_kernel<16>, grid, dim3(64), 0, s, x, splits, n, y, h);
         else hipLaunchKernelGGL(sum_cols_kernel<24>, grid, dim3(64), 0, s, x, splits, n, y, h);

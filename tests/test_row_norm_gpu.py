@@ -63,6 +63,6 @@ def test_add_rmsnorm_bounds(splits, n, hidden):
                                          (17, 1, 16380), (17, 1, 16384), (24, 2, 8196), (25, 3, 5464), (8, 3, 2048), (8, 2, 32764),
                                          (8, 2, 32768), (17, 3, 5460), (5, 128, 4092),
                                          (5, 128, 4096), (17, 128, 4096), (64, 46, 1280), (65, 46, 1280), (65, 7, 37444),
-                                         (65, 7, 37452)])
+                                         (65, 7, 37452), (8, 20, 3276), (8, 20, 3280), (12, 20, 5120)])
 def test_sum_parts_bounds(splits, n, ld):
     test_sum_parts_sizes(splits, n, ld)
